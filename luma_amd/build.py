@@ -16,10 +16,14 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
-SOURCES = [os.path.join(HERE, "csrc", "luma_step.hip")]
+# (source, units): luma_step.hip is compiled once per LUMA_UNIT, side by side
+# (its fast kernels take 1 to 4 minutes each)
+SOURCES = [(os.path.join(HERE, "csrc", "luma_step.hip"), (3, 2, 1, 0))]
 
 OUT = os.path.join(HERE, "libluma_hip.so")
 HOST_SOURCE = os.path.join(HERE, "csrc", "luma_host.cpp")
@@ -27,7 +31,7 @@ HOST_OUT = os.path.join(HERE, "_luma_host" + sysconfig.get_config_var("EXT_SUFFI
 ARCH = os.environ.get("LUMA_OFFLOAD_ARCH", "gfx950")
 
 FLAGS = [
-    "-O3", "-std=c++17", "-fPIC", "-shared",
+    "-O3", "-std=c++17", "-fPIC",
     f"--offload-arch={ARCH}",
     "-ffp-contract=off",
     "-fhip-fp32-correctly-rounded-divide-sqrt",
@@ -74,8 +78,15 @@ def host_command():
 def build(verbose: bool = False) -> str:
     """Compile every HIP source into luma_amd/libluma_hip.so and the host
     module into luma_amd/_luma_host*.so; returns the library's path."""
-    _run([hipcc(), *FLAGS, *SOURCES], "hipcc", OUT, verbose)
-    _run(host_command(), "g++ (host module)", HOST_OUT, verbose)
+    cc = hipcc()
+    with tempfile.TemporaryDirectory(prefix="luma_build_") as tmp:
+        jobs = [([cc, *FLAGS, f"-DLUMA_UNIT={u}", "-c", src], "hipcc",
+                 os.path.join(tmp, f"{os.path.basename(src)}.{u}.o"), verbose)
+                for src, units in SOURCES for u in units]
+        jobs.append((host_command(), "g++ (host module)", HOST_OUT, verbose))
+        with ThreadPoolExecutor(max_workers=len(jobs)) as pool:
+            built = [f.result() for f in [pool.submit(_run, *j) for j in jobs]]
+        _run([cc, *FLAGS, "-shared", *built[:-1]], "hipcc (link)", OUT, verbose)
     return OUT
 
 

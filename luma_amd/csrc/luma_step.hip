@@ -26,6 +26,17 @@
 // exact codes land there before the codes go to HBM, and it streams the
 // gradients, parameters and preconditioner codes non-temporally so that L2
 // holds the momentum code lines.
+//
+// The fast kernels take minutes to compile (every gradient type, momentum
+// regime and scaling of a pass is one kernel), so the build compiles this
+// file once per unit, in parallel: LUMA_UNIT 0 holds the C ABI and the other
+// kernels, 1 the fast pass 1, 2 the fast pass 2, 3 the fast pass 2 with
+// injected uniforms.  Without LUMA_UNIT one object holds everything.
+#ifdef LUMA_UNIT
+#define LUMA_IN_UNIT(n) (LUMA_UNIT == (n))
+#else
+#define LUMA_IN_UNIT(n) 1
+#endif
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -103,6 +114,15 @@ struct StepSrc {
   int32_t medium_from;   // chunks from here on (to small_from): medium tensors
   int32_t reserved;
 };
+
+// Launches of the fast kernels, each defined in its kernel's unit.
+#define LUMA_LOCAL __attribute__((visibility("hidden")))
+LUMA_LOCAL void launch_pass1_fast(int32_t blocks, hipStream_t s, const StepSrc &src,
+                                  float *partials);
+LUMA_LOCAL void launch_pass2_fast(int32_t blocks, hipStream_t s, const StepSrc &src,
+                                  uint64_t base_seed);
+LUMA_LOCAL void launch_pass2_fast_injected(int32_t blocks, hipStream_t s, const StepSrc &src,
+                                           uint64_t base_seed);
 
 // How a chunk's elements are shared out: among nt threads (kThreads, a whole
 // workgroup; or 64, one wavefront of a medium record), tid this thread's
@@ -426,6 +446,7 @@ __device__ __host__ inline int32_t finalize_waves(const StepSrc &src, int32_t n_
   return n_tensors + (src.tensors ? (src.n_chunks + 63) / 64 : 0);
 }
 
+#if LUMA_IN_UNIT(0)
 __global__ __launch_bounds__(kThreads) void finalize_kernel(StepSrc src,
                                                             const float *__restrict__ partials,
                                                             int32_t n_tensors) {
@@ -468,6 +489,7 @@ __global__ __launch_bounds__(kThreads) void finalize_kernel(StepSrc src,
   finalize_tail(src, T, src.groups[T.group], prev, am, av, seed_at(cm, om, src.chunk_shift),
                 seed_at(cv, ov, src.chunk_shift));
 }
+#endif
 
 // The record of a chunk whose threads hold (am, im), (av, iv): the share's
 // argmax (a workgroup's, with barriers, or a wavefront's), put by its
@@ -497,6 +519,7 @@ __device__ __forceinline__ void element_ema(const Tensor &T, const Hyper &h, con
   exact_ema(m, v, g, h, mn, vn);
 }
 
+#if LUMA_IN_UNIT(0)
 __global__ __launch_bounds__(kThreads) void pass1_exact_kernel(StepSrc src,
                                                                float *__restrict__ partials) {
   if (skip_step(src)) return;
@@ -534,6 +557,7 @@ __global__ __launch_bounds__(kThreads) void pass1_exact_kernel(StepSrc src,
   }
   put_chunk(partials, rec, sh, am, av, im, iv);
 }
+#endif
 
 // ---------------------------------------------------------------------------
 //  Small tensors: one wavefront per chunk
@@ -603,11 +627,13 @@ __device__ __forceinline__ void pass1_small_body(const StepSrc &src, float *part
   if (lane == 0) put_partial(partials, cidx, am, av, im, iv);
 }
 
+#if LUMA_IN_UNIT(0)
 __global__ __launch_bounds__(kThreads) void pass1_small_kernel(StepSrc src,
                                                                float *__restrict__ partials) {
   if (skip_step(src)) return;
   pass1_small_body(src, partials, small_wave(blockIdx.x));
 }
+#endif
 
 // The exact pass 2 of elements e0 .. min(e0 + 8, end) - 1: update, draws
 // (Philox or injected), new codes.
@@ -642,6 +668,7 @@ __device__ __forceinline__ void exact_group(const Tensor &T, const Hyper &h, con
   }
 }
 
+#if LUMA_IN_UNIT(0)
 __global__ __launch_bounds__(kThreads) void pass2_exact_kernel(StepSrc src, uint64_t base_seed,
                                                                int noise_mode) {
   if (skip_step(src)) return;
@@ -667,6 +694,7 @@ __global__ __launch_bounds__(kThreads) void pass2_exact_kernel(StepSrc src, uint
   for (int64_t e0 = beg + (int64_t)sh.tid() * kVec; e0 < end; e0 += (int64_t)sh.nt * kVec)
     exact_group(T, h, old, G, e0, end, scaled, inv, inj, pb, k0, k1);
 }
+#endif
 
 // Pass 2 of small wavefront w through the exact path (the exact-only mode's
 // kernel; the fast pass 2 steps small tensors like medium ones).
@@ -729,11 +757,13 @@ __device__ __forceinline__ void pass2_small_body(const StepSrc &src, uint64_t ba
   }
 }
 
+#if LUMA_IN_UNIT(0)
 __global__ __launch_bounds__(kThreads) void pass2_small_kernel(StepSrc src, uint64_t base_seed,
                                                                int noise_mode) {
   if (skip_step(src)) return;
   pass2_small_body(src, base_seed, noise_mode, small_wave(blockIdx.x));
 }
+#endif
 
 // ---------------------------------------------------------------------------
 //  Fast path: 8 consecutive elements per thread per iteration, 16-byte
@@ -1541,6 +1571,7 @@ __device__ __forceinline__ bool summaries_valid(const Tensor &T, const LUMA_GLOB
          __builtin_isfinite(old->fast[kIwmin]) && tensor_vec_ok(T);
 }
 
+#if LUMA_IN_UNIT(1)
 __global__ __launch_bounds__(kThreads, 4) void pass1_fast_kernel(StepSrc src,
                                                               float *__restrict__ partials) {
   if (skip_step(src)) return;
@@ -1596,6 +1627,11 @@ __global__ __launch_bounds__(kThreads, 4) void pass1_fast_kernel(StepSrc src,
                                   exi_m, exi_v, q, sh);
   put_chunk(partials, rec, sh, exm, exv, exi_m, exi_v);
 }
+
+void launch_pass1_fast(int32_t blocks, hipStream_t s, const StepSrc &src, float *partials) {
+  hipLaunchKernelGGL(pass1_fast_kernel, dim3(blocks), dim3(kThreads), 0, s, src, partials);
+}
+#endif
 
 // Inclusive prefix sum over the 64 lanes of a wave (all lanes active): three
 // row shifts of the original value, shifts by 4 and 8 within rows, then
@@ -2361,6 +2397,22 @@ __global__ __launch_bounds__(kThreads) void pass2_fast_kernel(StepSrc src, uint6
                                           reg, q, sh);
 }
 
+#if LUMA_IN_UNIT(2)
+void launch_pass2_fast(int32_t blocks, hipStream_t s, const StepSrc &src, uint64_t base_seed) {
+  hipLaunchKernelGGL(pass2_fast_kernel<false>, dim3(blocks), dim3(kThreads), 0, s, src, base_seed,
+                     (int)LUMA_NOISE_PHILOX);
+}
+#endif
+
+#if LUMA_IN_UNIT(3)
+void launch_pass2_fast_injected(int32_t blocks, hipStream_t s, const StepSrc &src,
+                                uint64_t base_seed) {
+  hipLaunchKernelGGL(pass2_fast_kernel<true>, dim3(blocks), dim3(kThreads), 0, s, src, base_seed,
+                     (int)LUMA_NOISE_INJECTED);
+}
+#endif
+
+#if LUMA_IN_UNIT(0)
 // ---------------------------------------------------------------------------
 //  Scale slots, decode (export) and quantise (import)
 // ---------------------------------------------------------------------------
@@ -2501,8 +2553,11 @@ __global__ void hyper_rows_kernel(LumaGroup g, int64_t t0, int n, float *__restr
   o[7] = h.eps;
 }
 
+#endif  // LUMA_IN_UNIT(0)
+
 }  // namespace luma
 
+#if LUMA_IN_UNIT(0)
 // ---------------------------------------------------------------------------
 //  C ABI
 // ---------------------------------------------------------------------------
@@ -2593,7 +2648,7 @@ static int launch_step(StepSrc src, int32_t n_tensors, int32_t n_chunks, float *
     if (exact)
       hipLaunchKernelGGL(pass1_exact_kernel, dim3(blocks), dim3(kThreads), 0, s, src, partials);
     else
-      hipLaunchKernelGGL(pass1_fast_kernel, dim3(fast_blocks), dim3(kThreads), 0, s, src, partials);
+      launch_pass1_fast(fast_blocks, s, src, partials);
     if (int r = check_launch("luma_step: pass 1 launch")) return r;
   }
   if (exact && small_blocks > 0) {
@@ -2614,11 +2669,9 @@ static int launch_step(StepSrc src, int32_t n_tensors, int32_t n_chunks, float *
       hipLaunchKernelGGL(pass2_exact_kernel, dim3(blocks), dim3(kThreads), 0, s, src, base_seed,
                          (int)noise_mode);
     else if (noise_mode == LUMA_NOISE_INJECTED)
-      hipLaunchKernelGGL(pass2_fast_kernel<true>, dim3(p2_blocks), dim3(kThreads), 0, s, src,
-                         base_seed, (int)noise_mode);
+      launch_pass2_fast_injected(p2_blocks, s, src, base_seed);
     else
-      hipLaunchKernelGGL(pass2_fast_kernel<false>, dim3(p2_blocks), dim3(kThreads), 0, s, src,
-                         base_seed, (int)noise_mode);
+      launch_pass2_fast(p2_blocks, s, src, base_seed);
     if (int r = check_launch("luma_step: pass 2 launch")) return r;
   }
   if (exact && small_blocks > 0) {
@@ -2801,3 +2854,4 @@ void luma_philox4x32(const uint32_t ctr[4], const uint32_t key[2], uint32_t out[
 }
 
 }  // extern "C"
+#endif  // LUMA_IN_UNIT(0)
