@@ -79,21 +79,31 @@ __device__ __forceinline__ float clamp_t(float x, float lo, float hi) {
 }
 
 // _precompute (functional.py:74-92) in double; K_M = 32767, K_W = 65535.
-__device__ inline void make_grid(double S_m, double S_v, double eps, Grid &g) {
-  const double w_min = 1.0 / (::sqrt(S_v) + eps);
+// The momentum half (from S_m) and the preconditioner half (from S_v) share
+// nothing, so the step's finalize derives them in two wavefronts.
+__device__ __forceinline__ void make_grid_m(double S_m, Grid &g) {
   const double delta_m = ::log1p(S_m) / 32767.0;
   const double z_m = ::expm1(delta_m);
+  g.dm = (float)delta_m;
+  g.zm = (float)z_m;
+  g.sm = (float)S_m;
+}
+
+__device__ __forceinline__ void make_grid_w(double S_v, double eps, Grid &g) {
+  const double w_min = 1.0 / (::sqrt(S_v) + eps);
   const double ratio = 1.0 / (eps * w_min);
   const double delta_w = ratio > 1.0 ? ::log(ratio) / 65535.0 : 0.0;
   const double z_w = delta_w > 0.0 ? ::expm1(delta_w) : 1.0;
-  g.dm = (float)delta_m;
-  g.zm = (float)z_m;
   g.wmin = (float)w_min;
   g.dw = (float)delta_w;
   g.zw = (float)z_w;
   g.wmax = (float)(1.0 / eps);
-  g.sm = (float)S_m;
   g.dwpos = delta_w > 0.0 ? 1 : 0;
+}
+
+__device__ inline void make_grid(double S_m, double S_v, double eps, Grid &g) {
+  make_grid_m(S_m, g);
+  make_grid_w(S_v, eps, g);
   for (int i = 0; i < 20; ++i) g.fast[i] = 0.0f;
 }
 

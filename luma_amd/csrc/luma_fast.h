@@ -243,19 +243,22 @@ __device__ __forceinline__ FastEma fast_ema(int qm, int qw, float g, float dm, f
 
 namespace luma {
 
-// Derived constants of a freshly computed grid (finalize, set_scales, import);
-// eps is the group's float32 eps.
-__device__ inline void make_fast(Grid &g, float eps) {
-  for (int i = 0; i < 20; ++i) g.fast[i] = 0.0f;
+// Derived constants of a freshly computed grid (finalize, set_scales, import),
+// its momentum and its preconditioner half; eps is the group's float32 eps.
+__device__ __forceinline__ void make_fast_m(Grid &g) {
   g.fast[kIdm] = (float)(1.0 / (double)g.dm);
   g.fast[kYTopM] = cr_log1p(g.sm) / g.dm;
+  g.fast[kXTopM] = 32767.0f * g.dm;
+}
+
+__device__ __forceinline__ void make_fast_w(Grid &g, float eps) {
   g.fast[kIwmin] = (float)(1.0 / (double)g.wmin);
   g.fast[kNl2dw] = g.dwpos ? (float)(-0.6931471805599453 / (double)g.dw) : 0.0f;
   g.fast[kYTopW] = g.dwpos ? cr_log(g.wmax / g.wmin) / g.dw : 0.0f;
-  g.fast[kXTopM] = 32767.0f * g.dm;
   g.fast[kXTopW] = 65535.0f * g.dw;
   const double iw = 1.0 / (double)g.wmin;
   g.fast[kW2] = (float)(iw * iw * (1.0 + 1e-6));
+  g.fast[kCwHi] = g.fast[kCwLo] = 0.0f;
   if (g.dwpos) {
     const double c = -0.6931471805599453 / (double)g.dw;
     int e;
@@ -266,6 +269,12 @@ __device__ inline void make_fast(Grid &g, float eps) {
   }
   g.fast[kWe] = (float)((double)g.wmin * (double)eps);
   g.fast[kXMin] = (float)((double)g.wmin / (double)g.wmax);
+}
+
+__device__ inline void make_fast(Grid &g, float eps) {
+  for (int i = 0; i < 20; ++i) g.fast[i] = 0.0f;
+  make_fast_m(g);
+  make_fast_w(g, eps);
 }
 
 // Error bounds of one tensor's fast path for one step (built per workgroup).

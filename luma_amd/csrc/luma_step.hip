@@ -353,30 +353,66 @@ __device__ __forceinline__ double py_max(double a, double floor_) { return floor
 // the step's scalars (functional.py:209-213, 262-264), and keep the maxima's
 // elements as the next step's seeds.
 //
-// The tail, by one lane: from the tensor's maxima and the elements holding
-// them (-1: none), everything after the reduction.
+// What bounds it is one dependent chain of float64 operations per tensor
+// (two powers, three logarithms, two expm1, about ten divisions), in a
+// launch that the rest of the step waits for.  The chain falls into three
+// that share nothing but the step count: the momentum scale and its half of
+// the grid, the preconditioner scale and its half, and the step's scalars.
+// Each takes a wavefront of the tensor's workgroup, so that the launch is
+// as long as the longest of them.  Kernel time with one wavefront for the
+// whole chain -> with three (medians of a kernel trace): one 4096x4096
+// tensor 7.96 -> 5.88 us, 52 tensors (0.8M elements) 6.84 -> 4.76 us, the
+// 148 GPT-2-small tensors 13.4 -> 6.7 us, 20,000 tensors 16.4 -> 11.1 us.
+constexpr int kFinRoles = 3;   // wavefronts of a finalize workgroup
+constexpr int kRoleM = 0, kRoleW = 1;   // (2: the scalars, and the step count)
+
+// One role's part for tensor T, by one lane: from the largest |m'| (kRoleM)
+// or v' (kRoleW) and the element that holds it (-1: none).
 __device__ __forceinline__ void finalize_tail(const StepSrc &src, const Tensor &T,
-                                              const LumaGroup &grp, int64_t prev, float am,
-                                              float av, int64_t seed_m, int64_t seed_v) {
-  const double s_m = py_max((double)am, 1e-9);  // SCALE_FLOOR_M (config.py:25)
-  const double s_v = py_max((double)av, 0.0);
+                                              const LumaGroup &grp, int64_t t, int role, float a,
+                                              int64_t seed) {
   LUMA_GLOBAL Slot &s = *T.slot;
-  const int64_t t = prev + 1;
   const int par = (int)(t & 1);
-  const Hyper h = step_hyper(grp, t);
-  s.s_m[par] = s_m;
-  s.s_v[par] = s_v;
+  LUMA_GLOBAL Grid &o = s.grid[par];
   Grid g;
-  make_grid(s_m, s_v, grp.eps, g);
-  make_fast(g, h.eps);
-  s.grid[par] = g;
-  s.hyp = h;
-  s.step = t;
-  // (only the kThreads-workgroup route writes summaries)
-  s.summ_step = (src.summaries && T.summary && T.first_chunk < src.medium_from) ? t : 0;
-  s.summ_shift = src.chunk_shift;
-  s.seed_m = seed_m;
-  s.seed_v = seed_v;
+  if (role == kRoleM) {
+    const double s_m = py_max((double)a, 1e-9);  // SCALE_FLOOR_M (config.py:25)
+    make_grid_m(s_m, g);
+    make_fast_m(g);
+    s.s_m[par] = s_m;
+    o.dm = g.dm;
+    o.zm = g.zm;
+    o.sm = g.sm;
+    o.fast[kIdm] = g.fast[kIdm];
+    o.fast[kYTopM] = g.fast[kYTopM];
+    o.fast[kXTopM] = g.fast[kXTopM];
+    s.seed_m = seed;
+  } else if (role == kRoleW) {
+    const double s_v = py_max((double)a, 0.0);
+    make_grid_w(s_v, grp.eps, g);
+    make_fast_w(g, (float)grp.eps);
+    s.s_v[par] = s_v;
+    o.wmin = g.wmin;
+    o.dw = g.dw;
+    o.zw = g.zw;
+    o.wmax = g.wmax;
+    o.dwpos = g.dwpos;
+    o.fast[kIwmin] = g.fast[kIwmin];
+    o.fast[kNl2dw] = g.fast[kNl2dw];
+    o.fast[kYTopW] = g.fast[kYTopW];
+    o.fast[kXTopW] = g.fast[kXTopW];
+    o.fast[kW2] = g.fast[kW2];
+    o.fast[kCwHi] = g.fast[kCwHi];
+    o.fast[kCwLo] = g.fast[kCwLo];
+    o.fast[kWe] = g.fast[kWe];
+    o.fast[kXMin] = g.fast[kXMin];
+    s.seed_v = seed;
+  } else {
+    s.hyp = step_hyper(grp, t);
+    // (only the kThreads-workgroup route writes summaries)
+    s.summ_step = (src.summaries && T.summary && T.first_chunk < src.medium_from) ? t : 0;
+    s.summ_shift = src.chunk_shift;
+  }
 }
 
 // The element a chunk record's offset word names (-1: none).
@@ -384,110 +420,122 @@ __device__ __forceinline__ int64_t seed_at(uint32_t chunk, uint32_t off, int32_t
   return (chunk == kNoArg || off == kNoArg) ? -1 : ((int64_t)chunk << shift) + off;
 }
 
-// One wavefront for tensor T (wave-uniform): each lane folds every 64th of
-// the tensor's records, 16 loads in flight (a tensor of a few thousand
-// chunks reads them in a few round trips), keeping the offset word of its
-// best record, which the winning lane then hands out.
-__device__ __forceinline__ void finalize_wave(const StepSrc &src, const Tensor &T,
-                                              const LumaGroup &grp, const float *partials) {
-  const int64_t prev = T.slot->step;   // (loaded while the records stream in)
-  const uint32_t lane = lane_id();
-  const int nch = (int)(((T.numel - 1) >> src.chunk_shift) + 1);
-  float am = 0.0f, av = 0.0f;
-  uint32_t cm = kNoArg, cv = kNoArg;   // chunk (within the tensor) of each maximum
-  uint32_t om = kNoArg, ov = kNoArg;   // its offset word
-  const vf4 *rec = (const vf4 *)(partials + kPartialWords * (int64_t)T.first_chunk);
-  auto fold = [&](const vf4 &r, int i) {
-    if (beats(r.x, am)) {
-      am = r.x;
-      cm = (uint32_t)i;
-      om = __float_as_uint(r.z);
-    }
-    if (beats(r.y, av)) {
-      av = r.y;
-      cv = (uint32_t)i;
-      ov = __float_as_uint(r.w);
-    }
-  };
-  constexpr int kInFlight = 16;
-  int i = (int)lane;
-  for (; i + (kInFlight - 1) * 64 < nch; i += kInFlight * 64) {
-    vf4 r[kInFlight];
-#pragma unroll
-    for (int k = 0; k < kInFlight; ++k) r[k] = rec[i + 64 * k];
-#pragma unroll
-    for (int k = 0; k < kInFlight; ++k) fold(r[k], i + 64 * k);
-  }
-  for (; i < nch; i += 64) fold(rec[i], i);
-  // the lane that read chunk c is c % 64; wave_argmax keeps the smallest
-  // chunk among equal maxima, which is that lane's own first best
-  wave_argmax(am, cm);
-  wave_argmax(av, cv);
-  om = (uint32_t)__shfl((int)om, (int)(cm & 63u), 64);
-  ov = (uint32_t)__shfl((int)ov, (int)(cv & 63u), 64);
-  if (lane == 0)
-    finalize_tail(src, T, grp, prev, am, av, seed_at(cm, om, src.chunk_shift),
-                  seed_at(cv, ov, src.chunk_shift));
-}
-
-// Tensors of at most kLaneChunks chunks take a lane each: 64 to a wavefront,
-// the float64 tail of 64 tensors side by side.  The others take a wavefront.
-constexpr int kLaneChunks = 4;
-
 __device__ __forceinline__ int tensor_chunks(const Tensor &T, int32_t shift) {
   return (int)(((T.numel - 1) >> shift) + 1);
 }
 
-// Waves [0, n_tensors): one tensor each (those of more than kLaneChunks
-// chunks; the others return at once); then, from a tensor table, one lane
-// per chunk record: the lane of a tensor's first record steps a tensor of at
-// most kLaneChunks chunks.
-__device__ __host__ inline int32_t finalize_waves(const StepSrc &src, int32_t n_tensors) {
-  return n_tensors + (src.tensors ? (src.n_chunks + 63) / 64 : 0);
+// A role's running maximum over a tensor's chunk records: the value, its
+// chunk (within the tensor) and that record's offset word.
+struct FinBest {
+  float a = 0.0f;
+  uint32_t c = kNoArg, o = kNoArg;
+  __device__ __forceinline__ void fold(const vf4 &r, int i, int role) {
+    const float x = role == kRoleM ? r.x : r.y;
+    if (beats(x, a)) {
+      a = x;
+      c = (uint32_t)i;
+      o = __float_as_uint(role == kRoleM ? r.z : r.w);
+    }
+  }
+};
+
+// One role's wavefront for tensor T (wave-uniform), which makes step t: each
+// lane folds every 64th of the tensor's records, 16 loads in flight (a
+// tensor of a few thousand chunks reads them in a few round trips), keeping
+// the offset word of its best record, which the winning lane then hands out.
+__device__ __forceinline__ void finalize_wave(const StepSrc &src, const Tensor &T,
+                                              const LumaGroup &grp, const float *partials,
+                                              int64_t t, int role) {
+  const uint32_t lane = lane_id();
+  FinBest b;
+  if (role == kRoleM || role == kRoleW) {
+    const int nch = tensor_chunks(T, src.chunk_shift);
+    const vf4 *rec = (const vf4 *)(partials + kPartialWords * (int64_t)T.first_chunk);
+    constexpr int kInFlight = 16;
+    int i = (int)lane;
+    for (; i + (kInFlight - 1) * 64 < nch; i += kInFlight * 64) {
+      vf4 r[kInFlight];
+#pragma unroll
+      for (int k = 0; k < kInFlight; ++k) r[k] = rec[i + 64 * k];
+#pragma unroll
+      for (int k = 0; k < kInFlight; ++k) b.fold(r[k], i + 64 * k, role);
+    }
+    for (; i < nch; i += 64) b.fold(rec[i], i, role);
+    // the lane that read chunk c is c % 64; wave_argmax keeps the smallest
+    // chunk among equal maxima, which is that lane's own first best
+    wave_argmax(b.a, b.c);
+    b.o = (uint32_t)__shfl((int)b.o, (int)(b.c & 63u), 64);
+  }
+  if (lane == 0)
+    finalize_tail(src, T, grp, t, role, b.a, seed_at(b.c, b.o, src.chunk_shift));
+}
+
+// Tensors of at most kLaneChunks chunks take a lane (of each role's
+// wavefront): 64 to a workgroup, the chains of 64 tensors side by side.  The
+// others take a workgroup.
+constexpr int kLaneChunks = 4;
+
+// Workgroups [0, tensor workgroups) take the tensors of more than
+// kLaneChunks chunks, tensor i in workgroup i modulo their number (at most
+// kFinTensorBlocks: a table of 20,000 tensors would otherwise launch as many
+// workgroups to find nothing to do); then, from a tensor table, 64 chunk
+// records to a workgroup: the lanes of a tensor's first record step a tensor
+// of at most kLaneChunks chunks.
+constexpr int32_t kFinTensorBlocks = 1024;
+
+__device__ __host__ inline int32_t finalize_tensor_blocks(int32_t n_tensors) {
+  return n_tensors < kFinTensorBlocks ? n_tensors : kFinTensorBlocks;
 }
 
 #if LUMA_IN_UNIT(0)
-__global__ __launch_bounds__(kThreads) void finalize_kernel(StepSrc src,
-                                                            const float *__restrict__ partials,
-                                                            int32_t n_tensors) {
+__global__ __launch_bounds__(kFinRoles * 64) void finalize_kernel(
+    StepSrc src, const float *__restrict__ partials, int32_t n_tensors) {
   if (skip_step(src)) return;
-  const int32_t w = __builtin_amdgcn_readfirstlane((int32_t)blockIdx.x * (kThreads / 64) +
-                                                   (int32_t)(threadIdx.x >> 6));
-  if (w < n_tensors) {
-    if (!src.tensors) {
-      finalize_wave(src, src.one, src.group, partials);
-      return;
+  const int role = __builtin_amdgcn_readfirstlane((int32_t)(threadIdx.x >> 6));
+  const int32_t tb = finalize_tensor_blocks(n_tensors);
+  // Every role reads the step count before the barrier; the third role's
+  // wavefront advances it after.  (All branches around a barrier are uniform
+  // over the workgroup.)
+  if ((int32_t)blockIdx.x < tb) {
+    // the lanes look at 64 of the workgroup's tensors at a time
+    for (int64_t base = blockIdx.x; base < n_tensors; base += 64 * (int64_t)tb) {
+      const int64_t i = base + (int64_t)lane_id() * tb;
+      uint64_t todo = __ballot(i < n_tensors &&
+                               (!src.tensors ||
+                                ((src.tensors[i].numel - 1) >> src.chunk_shift) >= kLaneChunks));
+      for (; todo != 0; todo &= todo - 1) {
+        const int32_t w = __builtin_amdgcn_readfirstlane(
+            (int32_t)(base + (int64_t)__builtin_ctzll(todo) * tb));
+        const Tensor T = src.tensors ? src.tensors[w] : src.one;
+        const LumaGroup grp = src.tensors ? src.groups[T.group] : src.group;
+        const int64_t t = T.slot->step + 1;
+        finalize_wave(src, T, grp, partials, t, role);
+        __syncthreads();
+        if (threadIdx.x == (kFinRoles - 1) * 64) T.slot->step = t;
+      }
     }
-    const Tensor T = src.tensors[w];
-    if (tensor_chunks(T, src.chunk_shift) <= kLaneChunks) return;   // a lane's (below)
-    finalize_wave(src, T, src.groups[T.group], partials);
     return;
   }
-  if (!src.tensors) return;
-  const int64_t r = (int64_t)(w - n_tensors) * 64 + lane_id();
-  if (r >= src.n_chunks) return;   // (no wave operations below)
-  const Tensor T = src.tensors[src.chunks[r].tensor];
-  // the tensor's first record, and few enough chunks for one lane
-  if (T.first_chunk != r || tensor_chunks(T, src.chunk_shift) > kLaneChunks) return;
-  const int64_t prev = T.slot->step;
-  const int nch = tensor_chunks(T, src.chunk_shift);
-  float am = 0.0f, av = 0.0f;
-  uint32_t cm = kNoArg, cv = kNoArg, om = kNoArg, ov = kNoArg;
-  for (int c = 0; c < nch; ++c) {
-    const vf4 x = ((const vf4 *)partials)[r + c];
-    if (beats(x.x, am)) {
-      am = x.x;
-      cm = (uint32_t)c;
-      om = __float_as_uint(x.z);
-    }
-    if (beats(x.y, av)) {
-      av = x.y;
-      cv = (uint32_t)c;
-      ov = __float_as_uint(x.w);
-    }
+  const int64_t r = (int64_t)((int32_t)blockIdx.x - tb) * 64 + lane_id();
+  Tensor T{};
+  int64_t t = 0;
+  if (r < src.n_chunks) {
+    T = src.tensors[src.chunks[r].tensor];
+    // the tensor's first record, and few enough chunks for one lane
+    if (T.first_chunk == r && tensor_chunks(T, src.chunk_shift) <= kLaneChunks)
+      t = T.slot->step + 1;
   }
-  finalize_tail(src, T, src.groups[T.group], prev, am, av, seed_at(cm, om, src.chunk_shift),
-                seed_at(cv, ov, src.chunk_shift));
+  if (t > 0) {
+    FinBest b;
+    if (role == kRoleM || role == kRoleW) {
+      const int nch = tensor_chunks(T, src.chunk_shift);
+      for (int c = 0; c < nch; ++c) b.fold(((const vf4 *)partials)[r + c], c, role);
+    }
+    finalize_tail(src, T, src.groups[T.group], t, role, b.a,
+                  seed_at(b.c, b.o, src.chunk_shift));
+  }
+  __syncthreads();
+  if (t > 0 && role == kFinRoles - 1) T.slot->step = t;
 }
 #endif
 
@@ -2656,9 +2704,10 @@ static int launch_step(StepSrc src, int32_t n_tensors, int32_t n_chunks, float *
     if (int r = check_launch("luma_step: pass 1 (small tensors) launch")) return r;
   }
   if (int r = mark(1)) return r;
-  const int32_t fin_waves = finalize_waves(src, n_tensors);
-  hipLaunchKernelGGL(finalize_kernel, dim3((fin_waves + kThreads / 64 - 1) / (kThreads / 64)),
-                     dim3(kThreads), 0, s, src, (const float *)partials, n_tensors);
+  const int32_t fin_blocks =
+      finalize_tensor_blocks(n_tensors) + (src.tensors ? (n_chunks + 63) / 64 : 0);
+  hipLaunchKernelGGL(finalize_kernel, dim3(fin_blocks), dim3(kFinRoles * 64), 0, s, src,
+                     (const float *)partials, n_tensors);
   if (int r = check_launch("luma_step: finalize launch")) return r;
   if (int r = mark(2)) return r;
   // the fast pass 2 steps the small tensors as it does the medium ones, one
