@@ -126,6 +126,19 @@ extern "C" {
 
 /* luma_step flags. */
 #define LUMA_FLAG_EXACT_ONLY 1 /* take the exact per-element path everywhere */
+/*
+ * Let the step give a small set more workgroups than it has chunk records: in
+ * a set of at most 2048 workgroup and medium records the medium ones take a
+ * workgroup each, and all of them are split into 2^luma_split_shift parts
+ * of down to LUMA_CHUNK_ELEMS_MIN elements, which then are the chunks (of the
+ * code summaries too).  The results do not depend on it.  `partials` then needs
+ * luma_workspace_bytes(n_chunks + LUMA_SPLIT_CHUNKS) (luma_step_tensor: plus
+ * LUMA_SPLIT_CHUNKS likewise; luma_step_noalloc's own workspace has the room,
+ * and beyond LUMA_NOALLOC_MAX_CHUNKS - LUMA_SPLIT_CHUNKS chunks it ignores
+ * the flag).  Without the flag every record is one chunk.
+ */
+#define LUMA_FLAG_SPLIT 2
+#define LUMA_SPLIT_CHUNKS 1024
 
 /* One parameter tensor taking part in a step. */
 typedef struct LumaTensor {
@@ -235,6 +248,12 @@ void luma_layout(int32_t out[8]);
 
 /* Bytes of workspace luma_step / luma_step_tensor / luma_quantize need for n_chunks chunks. */
 size_t luma_workspace_bytes(int32_t n_chunks);
+
+/*
+ * How far LUMA_FLAG_SPLIT splits `records` workgroup and medium records of
+ * chunk_elems elements (luma_step: n_chunks - small_chunks): log2 of the parts.
+ */
+int32_t luma_split_shift(int32_t records, int32_t chunk_elems);
 
 /* Summary words a tensor of numel elements needs for chunks of chunk_elems elements. */
 int64_t luma_summary_words(int64_t numel, int32_t chunk_elems);

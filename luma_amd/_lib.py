@@ -29,6 +29,8 @@ ABI_VERSION = 9              # LUMA_ABI_VERSION
 GRAD_F32, GRAD_BF16, GRAD_F16 = 0, 1, 2
 NOISE_PHILOX, NOISE_INJECTED = 0, 1
 FLAG_EXACT_ONLY = 1
+FLAG_SPLIT = 2               # LUMA_FLAG_SPLIT
+SPLIT_CHUNKS = 1024          # LUMA_SPLIT_CHUNKS: workspace chunks it may add
 
 TENSOR_DTYPE = np.dtype([
     ("param", "<u8"), ("grad", "<u8"), ("q_m", "<u8"), ("q_w", "<u8"),
@@ -84,6 +86,7 @@ _SIGNATURES = {
     "luma_last_error": (ctypes.c_char_p, []),
     "luma_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int32]),
     "luma_summary_words": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int32]),
+    "luma_split_shift": (ctypes.c_int32, [ctypes.c_int32, ctypes.c_int32]),
     "luma_layout": (None, [ctypes.POINTER(ctypes.c_int32)]),
     "luma_step": (ctypes.c_int, [ctypes.POINTER(StepArgs), _VP]),
     "luma_step_noalloc": (ctypes.c_int, [ctypes.POINTER(StepArgs), _VP]),

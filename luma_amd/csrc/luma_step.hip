@@ -100,6 +100,12 @@ static_assert(sizeof(Tensor) == sizeof(LumaTensor), "tensor layout");
 // kernels' workgroups from medium_from on step four such records, one per
 // wavefront, through the same code), [small_from, n_chunks) the
 // wavefront-per-tensor exact kernels (small tensors).
+//
+// A launch may split every workgroup record into 2^split parts of 2^wg_shift
+// elements, a workgroup each (split_records): the part is then the chunk that
+// the kernels work on, and parts past the tensor's end have no workgroup's
+// work.  Wavefront records are never split.  part_record numbers the parts
+// and the wavefront records in one row: their places in `partials`.
 struct StepSrc {
   const Tensor *tensors;
   const LumaChunk *chunks;
@@ -112,6 +118,8 @@ struct StepSrc {
   int32_t small_from;    // chunks from here on: small tensors, one wavefront each
   int32_t n_chunks;
   int32_t medium_from;   // chunks from here on (to small_from): medium tensors
+  int32_t split;         // log2 of the parts of a workgroup record
+  int32_t wg_shift;      // log2 of a part's length: chunk_shift - split
   int32_t reserved;
 };
 
@@ -136,11 +144,27 @@ struct Share {
   }
 };
 
-// Elements [beg, end) of chunk ci of tensor T.
-__device__ __forceinline__ void chunk_range(const StepSrc &src, const Tensor &T, int64_t ci,
+// log2 of the chunk length that the threads of `sh` work on, and that of
+// every chunk of tensor T (its records lie in one run).
+__device__ __forceinline__ int32_t share_shift(const StepSrc &src, const Share &sh) {
+  return sh.nt == kThreads ? src.wg_shift : src.chunk_shift;
+}
+
+__device__ __forceinline__ int32_t tensor_shift(const StepSrc &src, const Tensor &T) {
+  return T.first_chunk < src.medium_from ? src.wg_shift : src.chunk_shift;
+}
+
+// The place in `partials` of record rec (of its first part).
+__device__ __forceinline__ int64_t part_record(const StepSrc &src, int64_t rec) {
+  const int64_t m = src.medium_from;
+  return rec < m ? rec << src.split : rec - m + (m << src.split);
+}
+
+// Elements [beg, end) of chunk ci (of 2^shift elements) of tensor T.
+__device__ __forceinline__ void chunk_range(int32_t shift, const Tensor &T, int64_t ci,
                                             int64_t &beg, int64_t &end) {
-  const int64_t len = (int64_t)1 << src.chunk_shift;
-  beg = ci << src.chunk_shift;
+  const int64_t len = (int64_t)1 << shift;
+  beg = ci << shift;
   end = beg + len < T.numel ? beg + len : T.numel;
 }
 
@@ -181,23 +205,29 @@ __device__ __forceinline__ float unscale_rt(float g, float inv, int dt) {
   return unscale<LUMA_GRAD_BF16>(g, inv);
 }
 
-// The chunk of this workgroup, or from medium_from on of this wavefront:
-// its record, tensor, group, chunk index and thread share.  False: the
-// wavefront has no record (the last workgroup of the wavefront run, which
+// The wavefront's number among those of the workgroups past the workgroup
+// records' (wave-uniform: the record and the tensor it names then load
+// through the scalar cache into scalar registers).
+__device__ __forceinline__ int32_t wave_number(const StepSrc &src) {
+  return __builtin_amdgcn_readfirstlane(
+      ((int32_t)blockIdx.x - (src.medium_from << src.split)) * (kThreads / 64) +
+      (int32_t)(threadIdx.x >> 6));
+}
+
+// The chunk of this workgroup (a part of a workgroup record), or past those
+// of this wavefront (a wavefront record): its tensor, group, chunk index and
+// thread share.  False: the workgroup's part lies past the tensor's end, or
+// the wavefront has no record (the last workgroup of the wavefront run, which
 // ends at small_from, or with to_end at the table's end).
 __device__ __forceinline__ bool chunk_job(const StepSrc &src, Tensor &T, LumaGroup &g,
-                                          int64_t &index, int64_t &rec, Share &sh,
-                                          bool to_end = false) {
+                                          int64_t &index, Share &sh, bool to_end = false) {
   if (src.tensors) {
-    if ((int32_t)blockIdx.x < src.medium_from) {
-      rec = blockIdx.x;
+    int32_t rec;
+    if ((int32_t)blockIdx.x < src.medium_from << src.split) {
+      rec = (int32_t)blockIdx.x >> src.split;
       sh = Share{kThreads};
     } else {
-      // wave-uniform (readfirstlane): the record and the tensor it names
-      // then load through the scalar cache into scalar registers
-      rec = __builtin_amdgcn_readfirstlane(
-          src.medium_from + (int32_t)(blockIdx.x - (uint32_t)src.medium_from) * (kThreads / 64) +
-          (int32_t)(threadIdx.x >> 6));
+      rec = src.medium_from + wave_number(src);
       if (rec >= (to_end ? src.n_chunks : src.small_from)) return false;
       sh = Share{64};
     }
@@ -205,30 +235,30 @@ __device__ __forceinline__ bool chunk_job(const StepSrc &src, Tensor &T, LumaGro
     T = src.tensors[c.tensor];
     g = src.groups[T.group];
     index = c.index;
+    if (sh.nt == kThreads && src.split != 0) {
+      index = (index << src.split) + (int64_t)(blockIdx.x & ((1u << src.split) - 1u));
+      return index << src.wg_shift < T.numel;
+    }
   } else {
     T = src.one;
     g = src.group;
-    index = rec = blockIdx.x;
+    index = blockIdx.x;
     sh = Share{kThreads};
   }
   return true;
 }
 
-// Workgroups of a pass-kernel launch: one per workgroup record, one per
-// four medium records.
-__device__ __host__ __forceinline__ int32_t pass_blocks(int32_t medium_from, int32_t small_from) {
-  return medium_from + (small_from - medium_from + kThreads / 64 - 1) / (kThreads / 64);
+// Its place in `partials`.
+__device__ __forceinline__ int64_t chunk_place(const StepSrc &src, const Share &sh) {
+  return sh.nt == kThreads ? (int32_t)blockIdx.x
+                           : (src.medium_from << src.split) + wave_number(src);
 }
 
-// The tensor of this workgroup (one workgroup per tensor).
-__device__ __forceinline__ void tensor_job(const StepSrc &src, Tensor &T, LumaGroup &g) {
-  if (src.tensors) {
-    T = src.tensors[blockIdx.x];
-    g = src.groups[T.group];
-  } else {
-    T = src.one;
-    g = src.group;
-  }
+// Workgroups of a pass-kernel launch: one per part of a workgroup record,
+// one per four wavefront records up to record `to`.
+__device__ __host__ __forceinline__ int32_t pass_blocks(const StepSrc &src, int32_t to) {
+  return (src.medium_from << src.split) +
+         (to - src.medium_from + kThreads / 64 - 1) / (kThreads / 64);
 }
 
 __device__ __forceinline__ float load_grad(const LUMA_GLOBAL void *g, int64_t i, int dt) {
@@ -411,7 +441,7 @@ __device__ __forceinline__ void finalize_tail(const StepSrc &src, const Tensor &
     s.hyp = step_hyper(grp, t);
     // (only the kThreads-workgroup route writes summaries)
     s.summ_step = (src.summaries && T.summary && T.first_chunk < src.medium_from) ? t : 0;
-    s.summ_shift = src.chunk_shift;
+    s.summ_shift = src.wg_shift;
   }
 }
 
@@ -449,8 +479,8 @@ __device__ __forceinline__ void finalize_wave(const StepSrc &src, const Tensor &
   const uint32_t lane = lane_id();
   FinBest b;
   if (role == kRoleM || role == kRoleW) {
-    const int nch = tensor_chunks(T, src.chunk_shift);
-    const vf4 *rec = (const vf4 *)(partials + kPartialWords * (int64_t)T.first_chunk);
+    const int nch = tensor_chunks(T, tensor_shift(src, T));
+    const vf4 *rec = (const vf4 *)partials + part_record(src, T.first_chunk);
     constexpr int kInFlight = 16;
     int i = (int)lane;
     for (; i + (kInFlight - 1) * 64 < nch; i += kInFlight * 64) {
@@ -467,7 +497,7 @@ __device__ __forceinline__ void finalize_wave(const StepSrc &src, const Tensor &
     b.o = (uint32_t)__shfl((int)b.o, (int)(b.c & 63u), 64);
   }
   if (lane == 0)
-    finalize_tail(src, T, grp, t, role, b.a, seed_at(b.c, b.o, src.chunk_shift));
+    finalize_tail(src, T, grp, t, role, b.a, seed_at(b.c, b.o, tensor_shift(src, T)));
 }
 
 // Tensors of at most kLaneChunks chunks take a lane (of each role's
@@ -500,9 +530,13 @@ __global__ __launch_bounds__(kFinRoles * 64) void finalize_kernel(
     // the lanes look at 64 of the workgroup's tensors at a time
     for (int64_t base = blockIdx.x; base < n_tensors; base += 64 * (int64_t)tb) {
       const int64_t i = base + (int64_t)lane_id() * tb;
-      uint64_t todo = __ballot(i < n_tensors &&
-                               (!src.tensors ||
-                                ((src.tensors[i].numel - 1) >> src.chunk_shift) >= kLaneChunks));
+      bool many = i < n_tensors;
+      if (many && src.tensors) {
+        const int32_t shift =
+            src.tensors[i].first_chunk < src.medium_from ? src.wg_shift : src.chunk_shift;
+        many = (src.tensors[i].numel - 1) >> shift >= kLaneChunks;
+      }
+      uint64_t todo = __ballot(many);
       for (; todo != 0; todo &= todo - 1) {
         const int32_t w = __builtin_amdgcn_readfirstlane(
             (int32_t)(base + (int64_t)__builtin_ctzll(todo) * tb));
@@ -522,17 +556,18 @@ __global__ __launch_bounds__(kFinRoles * 64) void finalize_kernel(
   if (r < src.n_chunks) {
     T = src.tensors[src.chunks[r].tensor];
     // the tensor's first record, and few enough chunks for one lane
-    if (T.first_chunk == r && tensor_chunks(T, src.chunk_shift) <= kLaneChunks)
+    if (T.first_chunk == r && tensor_chunks(T, tensor_shift(src, T)) <= kLaneChunks)
       t = T.slot->step + 1;
   }
   if (t > 0) {
     FinBest b;
     if (role == kRoleM || role == kRoleW) {
-      const int nch = tensor_chunks(T, src.chunk_shift);
-      for (int c = 0; c < nch; ++c) b.fold(((const vf4 *)partials)[r + c], c, role);
+      const int nch = tensor_chunks(T, tensor_shift(src, T));
+      const vf4 *rec = (const vf4 *)partials + part_record(src, r);
+      for (int c = 0; c < nch; ++c) b.fold(rec[c], c, role);
     }
     finalize_tail(src, T, src.groups[T.group], t, role, b.a,
-                  seed_at(b.c, b.o, src.chunk_shift));
+                  seed_at(b.c, b.o, tensor_shift(src, T)));
   }
   __syncthreads();
   if (t > 0 && role == kFinRoles - 1) T.slot->step = t;
@@ -573,9 +608,9 @@ __global__ __launch_bounds__(kThreads) void pass1_exact_kernel(StepSrc src,
   if (skip_step(src)) return;
   Tensor T;
   LumaGroup grp;
-  int64_t ci, rec;
+  int64_t ci;
   Share sh;
-  if (!chunk_job(src, T, grp, ci, rec, sh)) return;   // (wave mode: no barriers below)
+  if (!chunk_job(src, T, grp, ci, sh)) return;   // (wave mode: no barriers below)
   const Hyper h = group_hyper(grp);
   const bool scaled = src.scaling.grad_scale != nullptr;
   const float inv = inv_scale(src);
@@ -583,7 +618,7 @@ __global__ __launch_bounds__(kThreads) void pass1_exact_kernel(StepSrc src,
   const int64_t prev = T.slot->step;
   const Grid *old = prev >= 1 ? (const Grid *)&T.slot->grid[prev & 1] : nullptr;
   int64_t beg, end;
-  chunk_range(src, T, ci, beg, end);
+  chunk_range(share_shift(src, sh), T, ci, beg, end);
 
   float am = 0.0f, av = 0.0f;
   uint32_t im = kNoArg, iv = kNoArg;
@@ -603,7 +638,7 @@ __global__ __launch_bounds__(kThreads) void pass1_exact_kernel(StepSrc src,
       }
     }
   }
-  put_chunk(partials, rec, sh, am, av, im, iv);
+  put_chunk(partials, chunk_place(src, sh), sh, am, av, im, iv);
 }
 #endif
 
@@ -652,7 +687,7 @@ __device__ __forceinline__ void pass1_small_body(const StepSrc &src, float *part
   const int64_t prev = T.slot->step;
   const Grid *old = prev >= 1 ? (const Grid *)&T.slot->grid[prev & 1] : nullptr;
   int64_t beg, end;
-  chunk_range(src, T, ci, beg, end);
+  chunk_range(src.chunk_shift, T, ci, beg, end);
   const uint32_t lane = lane_id();
   float am = 0.0f, av = 0.0f;
   uint32_t im = kNoArg, iv = kNoArg;
@@ -672,7 +707,7 @@ __device__ __forceinline__ void pass1_small_body(const StepSrc &src, float *part
   }
   wave_argmax(am, im);
   wave_argmax(av, iv);
-  if (lane == 0) put_partial(partials, cidx, am, av, im, iv);
+  if (lane == 0) put_partial(partials, part_record(src, cidx), am, av, im, iv);
 }
 
 #if LUMA_IN_UNIT(0)
@@ -722,9 +757,9 @@ __global__ __launch_bounds__(kThreads) void pass2_exact_kernel(StepSrc src, uint
   if (skip_step(src)) return;
   Tensor T;
   LumaGroup grp;
-  int64_t ci, rec;
+  int64_t ci;
   Share sh;
-  if (!chunk_job(src, T, grp, ci, rec, sh)) return;
+  if (!chunk_job(src, T, grp, ci, sh)) return;
   const bool scaled = src.scaling.grad_scale != nullptr;
   const float inv = inv_scale(src);
   const Slot &S = *(const Slot *)T.slot;
@@ -733,7 +768,7 @@ __global__ __launch_bounds__(kThreads) void pass2_exact_kernel(StepSrc src, uint
   const Grid *old = t >= 2 ? &S.grid[(t - 1) & 1] : nullptr;
   const Grid G = S.grid[t & 1];
   int64_t beg, end;
-  chunk_range(src, T, ci, beg, end);
+  chunk_range(share_shift(src, sh), T, ci, beg, end);
   uint32_t k0, k1;
   step_key(base_seed, t, T.param_id, k0, k1);
   const PhiloxBase pb = philox_base(T.elem_offset);
@@ -760,7 +795,7 @@ __device__ __forceinline__ void pass2_small_body(const StepSrc &src, uint64_t ba
   const Grid *old = t >= 2 ? &S.grid[(t - 1) & 1] : nullptr;
   const Grid G = S.grid[t & 1];
   int64_t beg, end;
-  chunk_range(src, T, ci, beg, end);
+  chunk_range(src.chunk_shift, T, ci, beg, end);
   uint32_t k0, k1;
   step_key(base_seed, t, T.param_id, k0, k1);
   const PhiloxBase pb = philox_base(T.elem_offset);
@@ -1438,6 +1473,7 @@ __device__ void pass1_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
   // n = 0), so the ballots and the queue length stay uniform across the wave;
   // a wave stops once all its groups lie past the end.
   int it = 0;
+  seed_thresholds();   // (once, here: a later call would keep the seeds' loads live)
   if (SUMM && n_whole > 0) {
     // This thread's summary word sw (written by the previous pass 2 for the
     // same thread of the same chunk) and, once, the decode of its code
@@ -1485,7 +1521,6 @@ __device__ void pass1_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
     // loop's latch with the buffers' loads in another order, and the wait
     // for the first buffer, placed for every path into the header, would
     // then also wait for the second.
-    seed_thresholds();
     const int n3 = n_whole - n_whole % 3;
     for (; it < n3; it += 3) {
       load_grads<GD>(T, group_at(it + 2), rc);
@@ -1504,7 +1539,6 @@ __device__ void pass1_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
     // current one again after the last whole group, so that every iteration
     // issues the same loads); group 0 was loaded above
     Raw8 &raw = ra;
-    seed_thresholds();
     for (; it < n_whole; ++it) {
       const int64_t e0 = beg + ((int64_t)it * nt + sh.tid()) * kVec;
       const int64_t en = end - e0 - kStride >= kVec ? e0 + kStride : e0;
@@ -1513,7 +1547,6 @@ __device__ void pass1_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
       take(e0, kVec, am, av);
     }
   }
-  if (n_whole == 0) seed_thresholds();
   for (; it < n_it; ++it) {
     // a wave whose groups all lie past the end is done (small tensors)
     if (beg + ((int64_t)it * nt + (sh.tid() & ~63u)) * kVec >= end) break;
@@ -1625,7 +1658,7 @@ __global__ __launch_bounds__(kThreads, 4) void pass1_fast_kernel(StepSrc src,
   if (skip_step(src)) return;
   {
     // workgroups past the workgroup and medium records: small tensors
-    const int32_t own = pass_blocks(src.medium_from, src.small_from);
+    const int32_t own = pass_blocks(src, src.small_from);
     if (src.tensors && (int32_t)blockIdx.x >= own) {
       pass1_small_body(src, partials, small_wave((int64_t)blockIdx.x - own));
       return;
@@ -1633,21 +1666,21 @@ __global__ __launch_bounds__(kThreads, 4) void pass1_fast_kernel(StepSrc src,
   }
   Tensor T;
   LumaGroup grp;
-  int64_t ci, rec;
+  int64_t ci;
   Share sh;
-  if (!chunk_job(src, T, grp, ci, rec, sh)) return;   // (wave mode: no barriers below)
+  if (!chunk_job(src, T, grp, ci, sh)) return;   // (wave mode: no barriers below)
   const Hyper h = group_hyper(grp);
   // this step is t = step + 1; its decode reads the grid of step t - 1
   const int64_t prev = T.slot->step;
   const LUMA_GLOBAL Grid *old = prev >= 1 ? &T.slot->grid[prev & 1] : nullptr;
   int64_t beg, end;
-  chunk_range(src, T, ci, beg, end);
+  chunk_range(share_shift(src, sh), T, ci, beg, end);
   const bool small = old == nullptr || old->fast[kXTopM] <= kSmall;
   const bool scaled = src.scaling.grad_scale != nullptr;
   const float inv = inv_scale(src);
   __shared__ uint32_t qbuf[kThreads / 64][kQueueCap];
   uint32_t *q = qbuf[threadIdx.x >> 6];
-  const bool summ = summaries_valid(T, old, prev, ci, src.chunk_shift, sh);
+  const bool summ = summaries_valid(T, old, prev, ci, share_shift(src, sh), sh);
   float exm = 0.0f, exv = 0.0f;
   uint32_t exi_m = kNoArg, exi_v = kNoArg;
   if (old == nullptr) {
@@ -1673,7 +1706,7 @@ __global__ __launch_bounds__(kThreads, 4) void pass1_fast_kernel(StepSrc src,
   else
     pass1_dispatch<LUMA_GRAD_F32>(T, h, old, inv, ci, beg, end, small, scaled, summ, exm, exv,
                                   exi_m, exi_v, q, sh);
-  put_chunk(partials, rec, sh, exm, exv, exi_m, exi_v);
+  put_chunk(partials, chunk_place(src, sh), sh, exm, exv, exi_m, exi_v);
 }
 
 void launch_pass1_fast(int32_t blocks, hipStream_t s, const StepSrc &src, float *partials) {
@@ -2412,17 +2445,17 @@ __global__ __launch_bounds__(kThreads) void pass2_fast_kernel(StepSrc src, uint6
   if (skip_step(src)) return;
   Tensor T;
   LumaGroup grp;
-  int64_t ci, rec;
+  int64_t ci;
   Share sh;
   // (the small tensors too: one wavefront each, after the medium ones)
-  if (!chunk_job(src, T, grp, ci, rec, sh, true)) return;   // (no barriers below)
+  if (!chunk_job(src, T, grp, ci, sh, true)) return;   // (no barriers below)
   const LUMA_GLOBAL Slot *S = T.slot;
   const int64_t t = S->step;   // advanced by finalize
   const Hyper h = S->hyp;
   const LUMA_GLOBAL Grid *old = t >= 2 ? &S->grid[(t - 1) & 1] : nullptr;
   const LUMA_GLOBAL Grid *nw = &S->grid[t & 1];
   int64_t beg, end;
-  chunk_range(src, T, ci, beg, end);
+  chunk_range(share_shift(src, sh), T, ci, beg, end);
   uint32_t k0, k1;
   step_key(base_seed, t, T.param_id, k0, k1);
   const bool inj = injected(T, noise_mode);
@@ -2650,6 +2683,37 @@ int64_t luma_summary_words(int64_t numel, int32_t chunk_elems) {
   return ((numel - 1) / chunk_elems + 1) * LUMA_SUMMARY_WORDS;
 }
 
+// A launch of about as many workgroups as the chip holds at once (768: three
+// to a CU, pass 2's registers) is as long as one workgroup, and a workgroup
+// as long as its iterations of 2,048 elements (about 2 us each in pass 2,
+// after 10 us of set-up and fallback): more and shorter parts are then free.
+// Parts of 8,192 elements while there are at most 1,024 of them, of 4,096 at
+// most 768, of 2,048 at most 384 (with more, pass 1 and finalize lose what
+// pass 2 gains).  Step times (us) by the part's length, 16,384 / 8,192 /
+// 4,096 / 2,048 elements:
+//   1 tensor of 200,000 (13 records)       37.9  28.7  25.3  25.4
+//   1 tensor of 1,000,003 (62)             39.0  29.3  26.1  27.9
+//   3 tensors, 2.2M elements (138)         42.5  39.7  36.6  45.2
+//   1 tensor of 4,185,079 (256)            45.4  44.5  46.2
+//   400 tensors, 4.1M elements (393)       60.9  53.7  57.5  69.4
+//   1 tensor of 12,500,000 (763)           82.3  90.0 109.0
+int32_t luma_split_shift(int32_t records, int32_t chunk_elems) {
+  if (records <= 0 || chunk_elems <= 0) return 0;
+  const int32_t shift = 31 - __builtin_clz((unsigned)chunk_elems);
+  const auto fits = [&](int32_t split) -> bool {
+    const int32_t part = shift - split;
+    const int64_t most = part >= 13   ? LUMA_SPLIT_CHUNKS
+                         : part == 12 ? LUMA_SPLIT_CHUNKS * 3 / 4
+                         : part == 11 ? LUMA_SPLIT_CHUNKS * 3 / 8
+                                      : 0;
+    return (int64_t)records << split <= most;
+  };
+  static_assert(LUMA_CHUNK_ELEMS_MIN == 1 << 11, "shortest part");
+  int32_t split = 0;
+  while (fits(split + 1)) ++split;
+  return split;
+}
+
 size_t luma_workspace_bytes(int32_t n_chunks) {
   return (size_t)(n_chunks > 0 ? n_chunks : 0) * kPartialWords * sizeof(float);
 }
@@ -2689,7 +2753,8 @@ static int launch_step(StepSrc src, int32_t n_tensors, int32_t n_chunks, float *
   // (the fast pass 1 runs the small tensors' exact pass 1 in workgroups past
   // its own, and the fast pass 2 steps them as it steps the medium ones; the
   // exact-only mode leaves them to the small kernels)
-  const int32_t blocks = pass_blocks(src.medium_from, src.small_from);
+  src.wg_shift = src.chunk_shift - src.split;
+  const int32_t blocks = pass_blocks(src, src.small_from);
   const int32_t small_blocks = (n_chunks - src.small_from + kThreads / 64 - 1) / (kThreads / 64);
   const int32_t fast_blocks = blocks + (src.tensors ? small_blocks : 0);
   if (exact ? blocks > 0 : fast_blocks > 0) {
@@ -2712,7 +2777,7 @@ static int launch_step(StepSrc src, int32_t n_tensors, int32_t n_chunks, float *
   if (int r = mark(2)) return r;
   // the fast pass 2 steps the small tensors as it does the medium ones, one
   // wavefront each in workgroups after theirs
-  const int32_t p2_blocks = pass_blocks(src.medium_from, src.tensors ? n_chunks : src.small_from);
+  const int32_t p2_blocks = pass_blocks(src, src.tensors ? n_chunks : src.small_from);
   if (exact ? blocks > 0 : p2_blocks > 0) {
     if (exact)
       hipLaunchKernelGGL(pass2_exact_kernel, dim3(blocks), dim3(kThreads), 0, s, src, base_seed,
@@ -2730,6 +2795,15 @@ static int launch_step(StepSrc src, int32_t n_tensors, int32_t n_chunks, float *
   }
   return mark(3);
 }
+
+// LUMA_FLAG_SPLIT: with at most this many workgroup and medium records, a
+// medium tensor takes a workgroup as the others do.  The wavefront route saves
+// a full chip's workgroup slots (20,000 tensors: pass 2 0.643 -> 0.616 ms with
+// it); on a chip that has slots to spare, one wavefront is only four times
+// slower than four (6 tensors, 11,441 elements: step 58.9 us by wavefronts,
+// 28.8 us by workgroups; 400 tensors, 588 records: 79.7 and 63.3 us; 2,000
+// tensors, 2,396 records: 134.7 and 132.1 us).
+constexpr int32_t kWideRecords = 2048;
 
 static int step_impl(const LumaStepArgs *a, void *stream, void *const *events) {
   if (!a) return fail("luma_step: null args");
@@ -2753,6 +2827,11 @@ static int step_impl(const LumaStepArgs *a, void *stream, void *const *events) {
   src.small_from = a->n_chunks - a->small_chunks;
   src.medium_from = src.small_from - a->medium_chunks;
   src.n_chunks = a->n_chunks;
+  if ((a->flags & LUMA_FLAG_SPLIT) != 0 && (a->flags & LUMA_FLAG_EXACT_ONLY) == 0 &&
+      src.small_from <= kWideRecords) {
+    src.medium_from = src.small_from;   // medium tensors: a workgroup each
+    src.split = luma_split_shift(src.small_from, c);
+  }
   return launch_step(src, a->n_tensors, a->n_chunks, a->partials, a->base_seed, a->noise_mode,
                      a->flags, static_cast<hipStream_t>(stream), events);
 }
@@ -2797,6 +2876,7 @@ int luma_step_noalloc(const LumaStepArgs *a, void *stream) {
   if (int r = scratch_for(static_cast<hipStream_t>(stream), &ws)) return r;
   LumaStepArgs b = *a;
   b.partials = ws;   // every chunk writes its record before finalize reads it
+  if (a->n_chunks > LUMA_NOALLOC_MAX_CHUNKS - LUMA_SPLIT_CHUNKS) b.flags &= ~LUMA_FLAG_SPLIT;
   return step_impl(&b, stream, nullptr);
 }
 
@@ -2817,8 +2897,12 @@ int luma_step_tensor(const LumaTensor *tensor, const LumaGroup *group, float *pa
   while (shift > __builtin_ctz((unsigned)LUMA_STEP_TENSOR_CHUNK_MIN) &&
          ((tensor->numel - 1) >> shift) + 1 < 4096)
     --shift;
-  const int64_t nch = ((tensor->numel - 1) >> shift) + 1;
+  int64_t nch = ((tensor->numel - 1) >> shift) + 1;
   if (nch > 0x7fffffff) return fail("luma_step_tensor: tensor too large");
+  if ((flags & LUMA_FLAG_SPLIT) != 0) {
+    shift -= luma_split_shift((int32_t)nch, 1 << shift);
+    nch = ((tensor->numel - 1) >> shift) + 1;
+  }
   StepSrc src{};
   memcpy(&src.one, tensor, sizeof(Tensor));
   src.one.first_chunk = 0;

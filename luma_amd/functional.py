@@ -110,14 +110,15 @@ def _luma_step_op(param: torch.Tensor, grad: torch.Tensor, Q_m: torch.Tensor,
     tt["grad_dtype"] = _GRAD_CODES[grad.dtype]
     gg = np.array([(lr, beta1, beta2, eps, weight_decay, 0.0)], dtype=L.GROUP_DTYPE)
     nch = (n + L.STEP_TENSOR_CHUNK_MIN - 1) // L.STEP_TENSOR_CHUNK_MIN   # at most this many chunks
-    partials = torch.empty(max(lib.luma_workspace_bytes(nch) // 4, 4), dtype=torch.float32,
-                           device=param.device)
+    partials = torch.empty(lib.luma_workspace_bytes(nch + L.SPLIT_CHUNKS) // 4,
+                           dtype=torch.float32, device=param.device)
     noise = L.NOISE_PHILOX if u_m is None else L.NOISE_INJECTED
     stream = torch.cuda.current_stream(param.device).cuda_stream
     scaling = L.Scaling(None if grad_scale is None else grad_scale.data_ptr(),
                         None if found_inf is None else found_inf.data_ptr())
     rc = lib.luma_step_tensor(tt.ctypes.data, gg.ctypes.data, partials.data_ptr(),
-                              base_seed & _MASK64, noise, L.FLAG_EXACT_ONLY if exact else 0,
+                              base_seed & _MASK64, noise,
+                              L.FLAG_EXACT_ONLY if exact else L.FLAG_SPLIT,
                               ctypes.byref(scaling), stream)
     L.check(rc, "luma_step_tensor")
 

@@ -91,6 +91,8 @@ _ARENA_ALIGN = 128   # int16 elements: every Q tensor starts on a 256-byte bound
 # Smallest tensor given code summaries: pass 1 reads them only in whole
 # iterations of a workgroup (256 threads x 8 elements).
 _SUMMARY_MIN = 2048
+# The limits of the wavefront routes that LUMA_FLAG_SPLIT's rule was measured with.
+_ROUTES = (L.SMALL_TENSOR, L.MEDIUM_TENSOR)
 
 
 def state_arena(params, device):
@@ -138,13 +140,15 @@ class _Engine:
         self._tensor_src = None      # (table array, chunk setting) last uploaded or matched
         self._numel_key = None       # bytes of its numel column and chunk layout (chunk table)
         self._first = None           # first_chunk column of that layout
-        self._chunk = L.CHUNK_ELEMS  # chunk length of the uploaded chunk table
+        self._record = L.CHUNK_ELEMS # chunk length of the uploaded chunk table
+        self._chunk = L.CHUNK_ELEMS  # that of the last launch (its parts, if split)
         self.chunk_elems = 0         # fixed chunk length (a power of two), 0: chunk_for's choice
         self.small_tensors = True    # step tensors of <= SMALL_TENSOR elements a wavefront each
         self._small_chunks = 0       # trailing chunk records of such tensors (uploaded table)
         self.medium_tensors = True   # step tensors of <= MEDIUM_TENSOR elements one wavefront
                                      # each (inside the fast kernels' launches)
         self._medium_chunks = 0      # the records of such tensors, before the small ones
+        self.split = True            # let the library split the records of a small set
         self._d_tensors = None
         self._table_cache = {}       # tensor-table bytes -> device copy (most recent last)
         self._ptr_cache = {}         # sequence number -> (table, (n, 2) grad and param
@@ -203,6 +207,24 @@ class _Engine:
             while c < L.CHUNK_ELEMS and c < int(big.max()):
                 c *= 2
         return c
+
+    def _splits(self) -> bool:
+        """Whether the library may split records (LUMA_FLAG_SPLIT): unless the
+        chunk length or a route was set by hand."""
+        return (self.split and not self.chunk_elems
+                and (self._small_limit(), self._medium_limit()) == _ROUTES)
+
+    def part(self, records: int, c: int) -> int:
+        """Length of the chunks that a launch of ``records`` workgroup and
+        medium records of c elements works on."""
+        return c >> self.lib.luma_split_shift(records, c) if self._splits() else c
+
+    def summary_chunk(self, numels: np.ndarray) -> int:
+        """Chunk length that a step over tensors of these sizes keeps code
+        summaries for."""
+        c = self.chunk_for(numels)
+        big = numels[numels > self._small_limit()]
+        return self.part(int(((big + c - 1) // c).sum()), c)
 
     def table(self, rows) -> np.ndarray:
         """Tensor table of rows: (param, grad, q_m, q_w, u_m, u_w, slot, param_id,
@@ -264,7 +286,10 @@ class _Engine:
                 raise self._capture_error("a param group's hyper-parameters")
             self._d_groups = self._upload(groups)
             self._group_key = gkey
-        need = max(self.lib.luma_workspace_bytes(n_chunks) // 4, 4)
+        self._chunk = self.part(n_chunks - self._small_chunks, self._record)
+        if self._splits():
+            flags |= L.FLAG_SPLIT
+        need = self.lib.luma_workspace_bytes(n_chunks + L.SPLIT_CHUNKS) // 4
         if self._partials is None or self._partials.numel() < need:
             if capturing:
                 raise self._capture_error("the chunk count")
@@ -278,7 +303,7 @@ class _Engine:
             chunks=self._d_chunks.data_ptr(), groups=self._d_groups.data_ptr(),
             partials=self._partials.data_ptr(),
             base_seed=base_seed & _MASK64, noise_mode=noise_mode, flags=flags,
-            chunk_elems=self._chunk, small_chunks=self._small_chunks,
+            chunk_elems=self._record, small_chunks=self._small_chunks,
             medium_chunks=self._medium_chunks,
             scaling=L.Scaling(scaling[0] or None, scaling[1] or None))
         if self.profile_events is None:
@@ -358,7 +383,7 @@ class _Engine:
             self._n_chunks = len(ch)
             self._small_chunks = n_small
             self._medium_chunks = n_medium
-            self._chunk = c
+            self._record = c
             self._numel_key = nkey
             self._first = first
         else:
@@ -890,8 +915,8 @@ class LUMA(Optimizer):
                 state["Q_m"] = qm
                 state["Q_w"] = qw
         # code summaries: SUMMARY_WORDS words per chunk at this step's chunk length
-        chunk = engine.chunk_for(np.fromiter((w[2].numel() for w in work), dtype=np.int64,
-                                             count=len(work)))
+        chunk = engine.summary_chunk(np.fromiter((w[2].numel() for w in work), dtype=np.int64,
+                                                 count=len(work)))
         # (a tensor below one whole 2048-element iteration, or stepped by a
         # single wavefront, never reads a summary: it gets none)
         least = max(_SUMMARY_MIN, engine._wave_limit() + 1)
