@@ -71,6 +71,16 @@ static_assert(LUMA_CHUNK_ELEMS_MIN % (kThreads * kVec) == 0,
 #endif
 typedef float vf4 __attribute__((ext_vector_type(4)));
 typedef uint32_t vu4 __attribute__((ext_vector_type(4)));
+// The same in a tensor's memory, which only its element type aligns: a
+// gradient that is a view of a packed bucket, or a parameter of a flat buffer,
+// may start anywhere.  The memory unit takes 16-byte accesses at any address
+// (they compile to the same instructions; a wavefront that starts in the
+// middle of a cache line touches one line more), so there is one form of the
+// loops for all.  With an element at a time for tensors off a 16-byte
+// boundary, 200 tensors (26M elements, float32 gradients packed) took
+// pass 1 120 us and pass 2 249 us; now 32 and 125.
+typedef float vf4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t vu4u __attribute__((ext_vector_type(4), aligned(2)));
 
 struct Tensor {
   LUMA_GLOBAL float *param;
@@ -913,13 +923,13 @@ struct Raw8 {
 
 template <int GD>
 __device__ __forceinline__ void load_raw(const Tensor &T, int64_t e0, Raw8 &r) {
-  r.qm = *(const LUMA_GLOBAL vu4 *)(T.q_m + e0);
-  r.qw = *(const LUMA_GLOBAL vu4 *)(T.q_w + e0);
+  r.qm = *(const LUMA_GLOBAL vu4u *)(T.q_m + e0);
+  r.qw = *(const LUMA_GLOBAL vu4u *)(T.q_w + e0);
   if (GD == LUMA_GRAD_F32) {
-    r.g0 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL float *)T.grad + e0));
-    r.g1 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL float *)T.grad + e0 + 4));
+    r.g0 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL float *)T.grad + e0));
+    r.g1 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL float *)T.grad + e0 + 4));
   } else {
-    r.g0 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL uint16_t *)T.grad + e0));
+    r.g0 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL uint16_t *)T.grad + e0));
   }
 }
 
@@ -946,50 +956,17 @@ __device__ __forceinline__ void unpack_raw(const Raw8 &r, Group8 &G) {
   }
 }
 
-// Load the codes and gradients of elements e0 .. e0+7 (n of them valid).
-// STREAM: the gradient and preconditioner-code vectors are loaded non-temporally.
-template <int GD, bool STREAM = false>
-__device__ __forceinline__ void load_group(const Tensor &T, int64_t e0, int n, bool vec, Group8 &G) {
-  if (vec) {
-    const vu4 a = *(const LUMA_GLOBAL vu4 *)(T.q_m + e0);
-    const vu4 b = STREAM ? load_stream((const LUMA_GLOBAL vu4 *)(T.q_w + e0)) : *(const LUMA_GLOBAL vu4 *)(T.q_w + e0);
-    unpack_i16(a.x, G.qm[0], G.qm[1]);
-    unpack_i16(a.y, G.qm[2], G.qm[3]);
-    unpack_i16(a.z, G.qm[4], G.qm[5]);
-    unpack_i16(a.w, G.qm[6], G.qm[7]);
-    unpack_u16(b.x, G.qw[0], G.qw[1]);
-    unpack_u16(b.y, G.qw[2], G.qw[3]);
-    unpack_u16(b.z, G.qw[4], G.qw[5]);
-    unpack_u16(b.w, G.qw[6], G.qw[7]);
-    if (GD == LUMA_GRAD_F32) {
-      const LUMA_GLOBAL vf4 *gp = (const LUMA_GLOBAL vf4 *)((const LUMA_GLOBAL float *)T.grad + e0);
-      const vf4 g0 = STREAM ? load_stream(gp) : gp[0];
-      const vf4 g1 = STREAM ? load_stream(gp + 1) : gp[1];
-      G.g[0] = g0.x; G.g[1] = g0.y; G.g[2] = g0.z; G.g[3] = g0.w;
-      G.g[4] = g1.x; G.g[5] = g1.y; G.g[6] = g1.z; G.g[7] = g1.w;
-    } else {
-      const LUMA_GLOBAL vu4 *gp = (const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL uint16_t *)T.grad + e0);
-      const vu4 gw = STREAM ? load_stream(gp) : gp[0];
-      G.g[0] = grad_lo<GD>(gw.x); G.g[1] = grad_hi<GD>(gw.x);
-      G.g[2] = grad_lo<GD>(gw.y); G.g[3] = grad_hi<GD>(gw.y);
-      G.g[4] = grad_lo<GD>(gw.z); G.g[5] = grad_hi<GD>(gw.z);
-      G.g[6] = grad_lo<GD>(gw.w); G.g[7] = grad_hi<GD>(gw.w);
-    }
-  } else {
+// Load the codes and gradients of elements e0 .. e0+7, of which n < 8 are
+// valid, one at a time.
+template <int GD>
+__device__ __forceinline__ void load_group(const Tensor &T, int64_t e0, int n, Group8 &G) {
 #pragma unroll
-    for (int j = 0; j < kVec; ++j) {
-      const bool ok = j < n;
-      G.qm[j] = ok ? (int)T.q_m[e0 + j] : 0;
-      G.qw[j] = (int)((ok ? (uint32_t)(uint16_t)T.q_w[e0 + j] : 0u) | kCodeFloat);
-      G.g[j] = ok ? load_grad(T.grad, e0 + j, GD) : 0.0f;
-    }
+  for (int j = 0; j < kVec; ++j) {
+    const bool ok = j < n;
+    G.qm[j] = ok ? (int)T.q_m[e0 + j] : 0;
+    G.qw[j] = (int)((ok ? (uint32_t)(uint16_t)T.q_w[e0 + j] : 0u) | kCodeFloat);
+    G.g[j] = ok ? load_grad(T.grad, e0 + j, GD) : 0.0f;
   }
-}
-
-__device__ __forceinline__ bool tensor_vec_ok(const Tensor &T) {
-  const uintptr_t bits = (uintptr_t)T.param | (uintptr_t)T.grad | (uintptr_t)T.q_m |
-                         (uintptr_t)T.q_w | (uintptr_t)T.u_m | (uintptr_t)T.u_w;
-  return (bits & 15u) == 0;
 }
 
 // Exact path for one element, kept out of line so that its float64 constants
@@ -1181,7 +1158,7 @@ __device__ __forceinline__ void unscale_group(Group8 &G, float inv) {
   for (int j = 0; j < kVec; ++j) G.g[j] = unscale<GD>(G.g[j], inv);
 }
 
-// FULL: the group is whole and aligned, and raw already holds its codes
+// FULL: the group is whole, and raw already holds its codes
 // and gradients; the iteration reloads raw with the group it will process
 // next (en: elements en .. en+7), so that the load overlaps this group's
 // arithmetic.
@@ -1288,7 +1265,7 @@ __device__ __forceinline__ void p1_iter(const Tensor &T, const P1Const &K, int64
     unpack_raw<GD>(raw, G);
     load_raw<GD>(T, en, raw);
   } else {
-    load_group<GD>(T, e0, n, false, G);
+    load_group<GD>(T, e0, n, G);
   }
   unscale_group<GD, SCALED>(G, K.inv);
   p1_compute<SMALL, PRUNE>(G, K, FULL ? kVec : n, Tm, Tv, am, av);
@@ -1299,10 +1276,10 @@ __device__ __forceinline__ void p1_iter(const Tensor &T, const P1Const &K, int64
 template <int GD>
 __device__ __forceinline__ void load_grads(const Tensor &T, int64_t e0, Raw8 &r) {
   if (GD == LUMA_GRAD_F32) {
-    r.g0 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL float *)T.grad + e0));
-    r.g1 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL float *)T.grad + e0 + 4));
+    r.g0 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL float *)T.grad + e0));
+    r.g1 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL float *)T.grad + e0 + 4));
   } else {
-    r.g0 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL uint16_t *)T.grad + e0));
+    r.g0 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL uint16_t *)T.grad + e0));
   }
 }
 
@@ -1328,7 +1305,7 @@ __device__ __forceinline__ void unpack_grads(const Raw8 &r, Group8 &G) {
 // others (in practice a few per chunk) go through the wave's queue to the
 // exact path.
 // SUMM: the tensor's code summaries of the previous step are valid (and
-// old != null, the tensor 16-byte aligned).  Then each whole-group
+// old != null).  Then each whole-group
 // iteration first bounds its block from the summary and the gradients, and
 // loads the block's codes only when some lane's bound reaches the
 // thresholds: most blocks cost their gradients alone.
@@ -1344,11 +1321,10 @@ __device__ void pass1_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
   static_assert(NT == kThreads || NT == 64, "a workgroup or one wavefront per chunk");
   const int64_t kStride = (int64_t)1 << it_shift;
   const int n_it = (int)((end - beg + kStride - 1) >> it_shift);
-  const bool vec_ok = tensor_vec_ok(T);
   // Iterations in which every lane's group is whole run in a loop of their
   // own that loads each group one iteration ahead (below).
   // (uniform: readfirstlane keeps the loop's group offsets in SGPRs)
-  const int n_whole = __builtin_amdgcn_readfirstlane(vec_ok ? (int)((end - beg) >> it_shift) : 0);
+  const int n_whole = __builtin_amdgcn_readfirstlane((int)((end - beg) >> it_shift));
   auto group_at = [&](int j) {
     return beg + ((int64_t)(j < n_whole ? j : n_whole - 1) * nt + sh.tid()) * kVec;
   };
@@ -1498,8 +1474,8 @@ __device__ void pass1_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
       Group8 G;
       unpack_grads<GD>(cur, G);
       unscale_group<GD, SCALED>(G, K.inv);
-      const vu4 a = *(const LUMA_GLOBAL vu4 *)(T.q_m + e0);
-      const vu4 b = *(const LUMA_GLOBAL vu4 *)(T.q_w + e0);
+      const vu4 a = *(const LUMA_GLOBAL vu4u *)(T.q_m + e0);
+      const vu4 b = *(const LUMA_GLOBAL vu4u *)(T.q_w + e0);
       unpack_i16(a.x, G.qm[0], G.qm[1]);
       unpack_i16(a.y, G.qm[2], G.qm[3]);
       unpack_i16(a.z, G.qm[4], G.qm[5]);
@@ -1576,7 +1552,7 @@ struct InitMax {
 // copy of the record stays in registers.
 template <int GD>
 __device__ __noinline__ InitMax pass1_init_scan(const LUMA_GLOBAL void *grad, int64_t beg,
-                                                int64_t end, bool vec_ok, Share sh) {
+                                                int64_t end, Share sh) {
   const int64_t kStride = (int64_t)sh.nt * kVec;
   Tensor T{};
   T.grad = grad;
@@ -1589,7 +1565,7 @@ __device__ __noinline__ InitMax pass1_init_scan(const LUMA_GLOBAL void *grad, in
     }
   };
   for (int64_t e0 = beg + (int64_t)sh.tid() * kVec; e0 < end; e0 += kStride) {
-    if (vec_ok && end - e0 >= kVec) {
+    if (end - e0 >= kVec) {
       Raw8 rw;
       load_grads<GD>(T, e0, rw);
       Group8 G;
@@ -1640,8 +1616,7 @@ __device__ __forceinline__ void pass1_dispatch(const Tensor &T, const Hyper &h,
 
 // Whether pass 1 may use chunk ci's code summaries: the previous step's
 // pass 2 wrote them with this chunk length (the slot records both), they
-// fit in the array, its grid is finite, and the tensor's streams are 16-byte
-// aligned (the whole-group loop).
+// fit in the array, and its grid is finite.
 __device__ __forceinline__ bool summaries_valid(const Tensor &T, const LUMA_GLOBAL Grid *old,
                                                 int64_t prev, int64_t ci, int32_t shift,
                                                 const Share &sh) {
@@ -1649,7 +1624,7 @@ __device__ __forceinline__ bool summaries_valid(const Tensor &T, const LUMA_GLOB
          (ci + 1) * LUMA_SUMMARY_WORDS <= T.summary_words &&
          old != nullptr && T.slot->summ_step == prev && T.slot->summ_shift == shift &&
          __builtin_isfinite(old->dm) && __builtin_isfinite(old->dw) &&
-         __builtin_isfinite(old->fast[kIwmin]) && tensor_vec_ok(T);
+         __builtin_isfinite(old->fast[kIwmin]);
 }
 
 #if LUMA_IN_UNIT(1)
@@ -1684,11 +1659,10 @@ __global__ __launch_bounds__(kThreads, 4) void pass1_fast_kernel(StepSrc src,
   float exm = 0.0f, exv = 0.0f;
   uint32_t exi_m = kNoArg, exi_v = kNoArg;
   if (old == nullptr) {
-    const bool vec_ok = tensor_vec_ok(T);
     const InitMax r =
-        T.grad_dtype == LUMA_GRAD_BF16  ? pass1_init_scan<LUMA_GRAD_BF16>(T.grad, beg, end, vec_ok, sh)
-        : T.grad_dtype == LUMA_GRAD_F16 ? pass1_init_scan<LUMA_GRAD_F16>(T.grad, beg, end, vec_ok, sh)
-                                        : pass1_init_scan<LUMA_GRAD_F32>(T.grad, beg, end, vec_ok, sh);
+        T.grad_dtype == LUMA_GRAD_BF16  ? pass1_init_scan<LUMA_GRAD_BF16>(T.grad, beg, end, sh)
+        : T.grad_dtype == LUMA_GRAD_F16 ? pass1_init_scan<LUMA_GRAD_F16>(T.grad, beg, end, sh)
+                                        : pass1_init_scan<LUMA_GRAD_F32>(T.grad, beg, end, sh);
     // unscaling is monotone in |g|: only the largest is unscaled
     float g = __uint_as_float(r.gb);
     if (scaled) g = unscale_rt(g, inv, T.grad_dtype);
@@ -1849,8 +1823,8 @@ __device__ __forceinline__ void launder(P2Const &C) {
   C.inv = in_vgpr(C.inv);
 }
 
-// One iteration of 8 consecutive elements.  FULL: all 8 valid and 16-byte
-// aligned (vector loads/stores, no masking).  Returns which codes need the
+// One iteration of 8 consecutive elements.  FULL: all 8 valid (vector
+// loads/stores, no masking).  Returns which codes need the
 // exact path (bit j: momentum code of element j, bit 8 + j: preconditioner
 // code); Q, W and top_w (block T_w) are kept for the queues.
 // STAGE (FULL only): the preconditioner codes go to *stage (LDS) instead
@@ -1905,20 +1879,20 @@ struct P2Raw {
 template <int GD>
 __device__ __forceinline__ void load_p2_grads(const Tensor &T, int64_t e0, Raw8 &r) {
   if (GD == LUMA_GRAD_F32) {
-    r.g0 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL float *)T.grad + e0));
-    r.g1 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL float *)T.grad + e0 + 4));
+    r.g0 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL float *)T.grad + e0));
+    r.g1 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL float *)T.grad + e0 + 4));
   } else {
-    r.g0 = load_stream((const LUMA_GLOBAL vu4 *)((const LUMA_GLOBAL uint16_t *)T.grad + e0));
+    r.g0 = load_stream((const LUMA_GLOBAL vu4u *)((const LUMA_GLOBAL uint16_t *)T.grad + e0));
   }
 }
 
 template <int GD>
 __device__ __forceinline__ void load_p2raw(const Tensor &T, int64_t e0, P2Raw &R) {
-  R.r.qm = *(const LUMA_GLOBAL vu4 *)(T.q_m + e0);
-  R.r.qw = load_stream((const LUMA_GLOBAL vu4 *)(T.q_w + e0));
+  R.r.qm = *(const LUMA_GLOBAL vu4u *)(T.q_m + e0);
+  R.r.qw = load_stream((const LUMA_GLOBAL vu4u *)(T.q_w + e0));
   if (GD != LUMA_GRAD_F32) load_p2_grads<GD>(T, e0, R.r);
-  R.p0 = load_stream((const LUMA_GLOBAL vf4 *)(T.param + e0));
-  R.p1 = load_stream((const LUMA_GLOBAL vf4 *)(T.param + e0 + 4));
+  R.p0 = load_stream((const LUMA_GLOBAL vf4u *)(T.param + e0));
+  R.p1 = load_stream((const LUMA_GLOBAL vf4u *)(T.param + e0 + 4));
 }
 
 // W: the words of the old codes and (bfloat16) gradients, for the queues.
@@ -1936,7 +1910,7 @@ __device__ __forceinline__ uint32_t p2_iter(const Tensor &T, const P2Const &C, i
     W.qw[0] = R.qw.x; W.qw[1] = R.qw.y; W.qw[2] = R.qw.z; W.qw[3] = R.qw.w;
     W.g[0] = R.g0.x; W.g[1] = R.g0.y; W.g[2] = R.g0.z; W.g[3] = R.g0.w;
   } else {
-    load_group<GD, true>(T, e0, n, false, Q);
+    load_group<GD>(T, e0, n, Q);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       W.qm[i] = pack_lo16((uint32_t)Q.qm[2 * i + 1], (uint32_t)Q.qm[2 * i]);
@@ -2029,8 +2003,8 @@ __device__ __forceinline__ uint32_t p2_iter(const Tensor &T, const P2Const &C, i
     vf4 p0, p1;
     p0.x = p[0]; p0.y = p[1]; p0.z = p[2]; p0.w = p[3];
     p1.x = p[4]; p1.y = p[5]; p1.z = p[6]; p1.w = p[7];
-    store_stream(p0, (LUMA_GLOBAL vf4 *)(T.param + e0));
-    store_stream(p1, (LUMA_GLOBAL vf4 *)(T.param + e0 + 4));
+    store_stream(p0, (LUMA_GLOBAL vf4u *)(T.param + e0));
+    store_stream(p1, (LUMA_GLOBAL vf4u *)(T.param + e0 + 4));
     // two codes per word: the low halves of om[2i] and om[2i + 1] (v_perm)
     vu4 a, b;
     a.x = __builtin_amdgcn_perm(om[1], om[0], 0x05040100u);
@@ -2041,11 +2015,11 @@ __device__ __forceinline__ uint32_t p2_iter(const Tensor &T, const P2Const &C, i
     b.y = __builtin_amdgcn_perm(ow[3], ow[2], 0x05040100u);
     b.z = __builtin_amdgcn_perm(ow[5], ow[4], 0x05040100u);
     b.w = __builtin_amdgcn_perm(ow[7], ow[6], 0x05040100u);
-    *(LUMA_GLOBAL vu4 *)(T.q_m + e0) = a;
+    *(LUMA_GLOBAL vu4u *)(T.q_m + e0) = a;
     if (STAGE)
       *stage = make_uint4(b.x, b.y, b.z, b.w);
     else
-      *(LUMA_GLOBAL vu4 *)(T.q_w + e0) = b;
+      *(LUMA_GLOBAL vu4u *)(T.q_w + e0) = b;
     acc_codes(acc, a, b);
   } else {
     int qa = 0;
@@ -2075,11 +2049,10 @@ __device__ void pass2_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
   // iteration covers nt * kVec = 1 << it_shift consecutive elements.
   const int nt = sh.nt;
   const int it_shift = __builtin_ctz((unsigned)nt) + 3;
-  const bool vec_ok = tensor_vec_ok(T);
   // Iterations in which every lane's group is whole stage their
   // preconditioner codes; before a slot is reused, the iteration it holds has
   // its queued entries run and is written back.
-  const int n_whole = vec_ok ? (int)((end - beg) >> it_shift) : 0;
+  const int n_whole = (int)((end - beg) >> it_shift);
   // Each iteration's vectors are loaded one iteration ahead, into two
   // buffers in a loop unrolled by two (copying a buffer whose loads are in
   // flight would make the copy wait for them); past the last whole group the
@@ -2313,7 +2286,7 @@ __device__ void pass2_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
     const int64_t e = beg + ((int64_t)j * nt + sh.tid()) * kVec;
     vu4 w;
     w.x = v.x; w.y = v.y; w.z = v.z; w.w = v.w;
-    store_stream(w, (LUMA_GLOBAL vu4 *)(T.q_w + e));
+    store_stream(w, (LUMA_GLOBAL vu4u *)(T.q_w + e));
   };
   // Every lane of a wave runs the same iterations (lanes past the end carry
   // n = 0), so the ballots and the queue lengths stay uniform across the wave;
@@ -2370,7 +2343,7 @@ __device__ void pass2_fast_body(const Tensor &T, const Hyper &h, const LUMA_GLOB
     Words4 W;
     U4 top_w{};
     P2Raw R;
-    const bool whole = vec_ok && n == kVec;
+    const bool whole = n == kVec;
     if (whole) load_p2raw<GD>(T, e0, R);
     const uint32_t flags =
         whole ? p2_iter<GD, INJ, REG, SCALED, true, false>(T, C, e0, n, R, k0, k1, Q, W, top_w,
