@@ -81,6 +81,7 @@ typedef uint32_t vu4 __attribute__((ext_vector_type(4)));
 // pass 1 120 us and pass 2 249 us; now 32 and 125.
 typedef float vf4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t vu4u __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t vu4a __attribute__((ext_vector_type(4), aligned(4), may_alias));   // floats' bits
 
 struct Tensor {
   LUMA_GLOBAL float *param;
@@ -300,8 +301,9 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 
 // Block-wide NaN-propagating max of two values; result valid in thread 0.
+template <int NT>   // threads of the workgroup
 __device__ __forceinline__ void block_max2(float &a, float &b) {
-  __shared__ float sa[kThreads / 64], sb[kThreads / 64];
+  __shared__ float sa[NT / 64], sb[NT / 64];
   a = wave_max(a);
   b = wave_max(b);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -311,7 +313,7 @@ __device__ __forceinline__ void block_max2(float &a, float &b) {
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int i = 1; i < (int)(blockDim.x >> 6); ++i) {
+    for (int i = 1; i < NT / 64; ++i) {
       a = nan_max(a, sa[i]);
       b = nan_max(b, sb[i]);
     }
@@ -2471,17 +2473,30 @@ void launch_pass2_fast_injected(int32_t blocks, hipStream_t s, const StepSrc &sr
 //  Scale slots, decode (export) and quantise (import)
 // ---------------------------------------------------------------------------
 
-// Writes the state of one slot: step count t, the scales of step t and its grid.
-__device__ void write_slot(Slot &s, int64_t t, double s_m, double s_v, double eps) {
+// Writes the state of one slot: step count t, the scales of step t and its
+// grid, as a momentum and a preconditioner half (separate words of the slot).
+__device__ void write_slot_m(Slot &s, int64_t t, double s_m) {
   const int par = (int)(t & 1);
   s.s_m[par] = s_m;
-  s.s_v[par] = s_v;
-  make_grid(s_m, s_v, eps, s.grid[par]);
-  make_fast(s.grid[par], (float)eps);
+  make_grid_m(s_m, s.grid[par]);
+  make_fast_m(s.grid[par]);
   s.step = t;
   s.summ_step = 0;   // codes written by other means: no summaries for them
   s.summ_shift = 0;
   s.seed_m = s.seed_v = -1;
+}
+
+__device__ void write_slot_w(Slot &s, int64_t t, double s_v, double eps) {
+  const int par = (int)(t & 1);
+  s.s_v[par] = s_v;
+  make_grid_w(s_v, eps, s.grid[par]);
+  make_fast_w(s.grid[par], (float)eps);
+  for (int i = kFastCount; i < 20; ++i) s.grid[par].fast[i] = 0.0f;
+}
+
+__device__ void write_slot(Slot &s, int64_t t, double s_m, double s_v, double eps) {
+  write_slot_m(s, t, s_m);
+  write_slot_w(s, t, s_v, eps);
 }
 
 __global__ void set_scales_kernel(const LumaScaleInit *__restrict__ items, int n) {
@@ -2521,74 +2536,326 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(const int16_t *__restr
   }
 }
 
-__global__ __launch_bounds__(kThreads) void quant_max_kernel(const float *__restrict__ m,
-                                                             const float *__restrict__ v, int64_t n,
-                                                             float *__restrict__ partials) {
-  const int64_t beg = (int64_t)blockIdx.x * kChunk;
-  const int64_t end = beg + kChunk < n ? beg + kChunk : n;
-  float am = 0.0f, av = 0.0f;
-  for (int64_t i = beg + threadIdx.x; i < end; i += kThreads) {
-    const float vi = v[i];
-    am = nan_max(am, fabsf(m[i]));
-    av = nan_max(av, (vi != vi || vi > 0.0f) ? vi : 0.0f);
+// Import's kernels: the max pass reads 8 bytes per element, the quantise pass
+// reads 8 and writes 4 (HBM; a copy reaches 5.2 TB/s).  With one workgroup per
+// 131,072 elements, every code on the exact path (about 500 VALU instructions
+// per element, float64) and clones of both inputs, nine tensors of 218M
+// elements took 8.49 ms; now 1.08 ms.  Of a 58.7M-element tensor's: max pass
+// 72 us (6.5 TB/s; 121 us with cached instead of non-temporal loads), quantise
+// 199 us (3.5 TB/s: some 700 VALU instructions per 8 elements and the late
+// 2-byte stores of the exact codes; 232 us with non-temporal loads, which the
+// exact path's second read of m and v then misses).
+
+// The max pass: workgroups of 1,024 threads that step over the tensor, as
+// many as the chip holds at once but at most two per LUMA_CHUNK_ELEMS
+// elements (their records, two floats each, fit luma_workspace_bytes).
+constexpr int kMaxThreads = 1024;
+constexpr int64_t kMaxBlocks = 512;
+
+// The largest |m| and v (negative v count as 0; a NaN wins) by their bits:
+// for values without a sign the order of floats is that of their bits, NaN
+// above infinity.  v is folded as a signed integer (the negative ones stay
+// below the 0 it starts from) and as an unsigned one, which is above
+// 0xFF800000 when a NaN with a sign was among them.
+__global__ __launch_bounds__(kMaxThreads) void quant_max_kernel(const float *__restrict__ m,
+                                                                const float *__restrict__ v,
+                                                                int64_t n,
+                                                                float *__restrict__ partials) {
+  uint32_t am = 0u, uv = 0u;
+  int32_t av = 0;
+  auto take = [&](uint32_t mi, uint32_t vi) {
+    am = max(am, mi & 0x7FFFFFFFu);
+    av = max(av, (int32_t)vi);
+    uv = max(uv, vi);
+  };
+  // (4 elements per lane, so that a wavefront's load is one run of 1 KB)
+  constexpr int kInFlight = 4;
+  int64_t e0 = ((int64_t)blockIdx.x * kMaxThreads + threadIdx.x) * 4;
+  const int64_t stride = (int64_t)gridDim.x * kMaxThreads * 4;
+  for (; e0 + (kInFlight - 1) * stride + 4 <= n; e0 += kInFlight * stride) {
+    vu4a a[kInFlight], b[kInFlight];
+#pragma unroll
+    for (int k = 0; k < kInFlight; ++k) {
+      a[k] = __builtin_nontemporal_load((const vu4a *)(m + e0 + k * stride));
+      b[k] = __builtin_nontemporal_load((const vu4a *)(v + e0 + k * stride));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < kInFlight; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) take(a[k][j], b[k][j]);
   }
-  block_max2(am, av);
+  for (; e0 + 4 <= n; e0 += stride) {
+    const vu4a a = *(const vu4a *)(m + e0), b = *(const vu4a *)(v + e0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) take(a[j], b[j]);
+  }
+  for (; e0 < n; ++e0)   // the tensor's last, partial group (one thread)
+    take(__float_as_uint(m[e0]), __float_as_uint(v[e0]));
+  float fm = __uint_as_float(am), fv = __uint_as_float(uv > 0xFF800000u ? uv : (uint32_t)av);
+  block_max2<kMaxThreads>(fm, fv);
   if (threadIdx.x == 0) {
-    partials[2 * (int64_t)blockIdx.x] = am;
-    partials[2 * (int64_t)blockIdx.x + 1] = av;
+    partials[2 * (int64_t)blockIdx.x] = fm;
+    partials[2 * (int64_t)blockIdx.x + 1] = fv;
   }
 }
 
-__global__ __launch_bounds__(64) void quant_finalize_kernel(const float *__restrict__ partials,
-                                                            int nch, Slot *__restrict__ slot,
-                                                            int64_t step, double eps) {
+// One workgroup: the tensor's scales from the chunks' maxima, then its grid,
+// the momentum half in the first wavefront and the preconditioner half in the
+// second (each a chain of float64 operations of a few us).
+__global__ __launch_bounds__(kThreads) void quant_finalize_kernel(
+    const float *__restrict__ partials, int nch, Slot *__restrict__ slot, int64_t step, double eps) {
   float am = 0.0f, av = 0.0f;
-  for (int i = threadIdx.x; i < nch; i += 64) {
-    am = nan_max(am, partials[2 * i]);
-    av = nan_max(av, partials[2 * i + 1]);
+#pragma unroll 8
+  for (int i = threadIdx.x; i < nch; i += kThreads) {
+    am = nan_max(am, partials[2 * (int64_t)i]);
+    av = nan_max(av, partials[2 * (int64_t)i + 1]);
   }
-  am = wave_max(am);
-  av = wave_max(av);
-  if (threadIdx.x == 0) write_slot(*slot, step, py_max((double)am, 1e-9), py_max((double)av, 0.0), eps);
+  block_max2<kThreads>(am, av);
+  __shared__ float top[2];
+  if (threadIdx.x == 0) {
+    top[0] = am;
+    top[1] = av;
+  }
+  __syncthreads();
+  const double s_m = py_max((double)top[0], 1e-9), s_v = py_max((double)top[1], 0.0);
+  if (threadIdx.x == 0)
+    write_slot_m(*slot, step, s_m);
+  else if (threadIdx.x == 64)
+    write_slot_w(*slot, step, s_v, eps);
 }
 
+constexpr int kQuantQueue = 1024;   // entries of a wavefront's queue of either kind (a power of two)
+static_assert(kQuantQueue >= 64 * kVec + 63, "an iteration's elements and a rest below 64");
+// Workgroups of the quantise pass: as many as the chip holds at once (four
+// wavefronts per SIMD), each with one run of whole iterations, so that their
+// queues are drained with less than 64 entries once per run.
+constexpr int64_t kQuantBlocks = 1024;
+
+// Per-tensor constants of import's fast path (see pass 2's).
+struct QuantConst {
+  float idm, hk2, hk3;            // 1/dm; -k2, 0.5 - k3
+  float cf, ch, cl, wmin, we, xmin;   // preconditioner: as P2Const
+  float nk7, hk8;                 // -k7, 0.5 - k8
+  float zoff;
+};
+
+// The code of element i from its exact candidates (exact_quant_*_pair) and
+// the top 16 bits of its uniform (`which`: 0 momentum, 1 preconditioner);
+// the low 8 bits are drawn, and the double expm1 runs, only where those
+// leave the decision open.
+template <bool INJ>
+__device__ __forceinline__ int quant_draw(int lo, int hi, float a, float z, int64_t i, int which,
+                                          const float *__restrict__ u, PhiloxBase pb, uint32_t k0,
+                                          uint32_t k1) {
+  uint32_t top = 0u;
+  float ulo, uhi;
+  if (INJ) {
+    ulo = uhi = u[i];
+  } else {
+    top = u4_half(philox_block((uint64_t)i, pb, which ? kBlockTopW : kBlockTopM, k0, k1),
+                  (int)(i & 7));
+    ulo = (float)(top << 8) * 0x1p-24f;
+    uhi = (float)((top << 8) | 0xFFu) * 0x1p-24f;
+  }
+  const CodePair c = unpack_pair(sr_resolve(lo, hi, a, z, ulo, uhi));
+  if (c.lo == c.hi) return c.lo;
+  const U4 low = philox_block((uint64_t)i, pb, kBlockLow, k0, k1);
+  const float x = (float)((top << 8) | u4_byte(low, 2 * (int)(i & 7) + which)) * 0x1p-24f;
+  return x < exact_sr_prob(c.a, z) ? c.hi : c.lo;
+}
+
+// One run [beg, end) per workgroup.  m and v are what a first step's pass 2
+// has after its EMA, so its fast encode and its certification apply as they
+// are (the bounds of make_bounds without an old grid); codes that they leave
+// open (about 1% of each kind) go to the wavefront's queues in LDS and are
+// computed on the exact path 64 at a time.
+template <bool INJ, int REG>
+__device__ __forceinline__ void quant_body(const float *__restrict__ m, const float *__restrict__ v,
+                                           int64_t beg, int64_t end, int16_t *q_m, int16_t *q_w,
+                                           const Grid &G, const QuantConst &C, float epsf,
+                                           uint32_t k0, uint32_t k1, const float *__restrict__ u_m,
+                                           const float *__restrict__ u_w, uint32_t *queue) {
+  const PhiloxBase pb{0, 0};
+  const uint32_t lane = lane_id();
+  uint32_t *queue_m = queue, *queue_w = queue + kQuantQueue;
+  uint32_t head_m = 0, len_m = 0;   // a queue's oldest entry and its length
+  uint32_t head_w = 0, len_w = 0;
+  const int n_it = (int)((end - beg + kThreads * kVec - 1) / (kThreads * kVec));
+  for (int it = 0; it <= n_it; ++it) {
+    // the last visit (it == n_it) only drains
+    const int64_t e0 = beg + ((int64_t)it * kThreads + threadIdx.x) * kVec;
+    const int64_t rem = it < n_it ? end - e0 : 0;
+    const int n = rem <= 0 ? 0 : (rem < kVec ? (int)rem : kVec);
+    uint32_t flags = 0;
+    if (n > 0) {
+      float mm[kVec], vv[kVec], zmu_m[kVec], zmu_w[kVec];
+      if (n == kVec) {
+        const vf4u m0 = *(const vf4u *)(m + e0), m1 = *(const vf4u *)(m + e0 + 4);
+        const vf4u v0 = *(const vf4u *)(v + e0), v1 = *(const vf4u *)(v + e0 + 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          mm[j] = m0[j];
+          mm[j + 4] = m1[j];
+          vv[j] = v0[j];
+          vv[j + 4] = v1[j];
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) {
+          mm[j] = j < n ? m[e0 + j] : 0.0f;
+          vv[j] = j < n ? v[e0 + j] : 0.0f;
+        }
+      }
+      if (INJ) {
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) {
+          zmu_m[j] = C.zoff - (j < n ? u_m[e0 + j] : 0.5f);
+          zmu_w[j] = C.zoff - (j < n ? u_w[e0 + j] : 0.5f);
+        }
+      } else {
+        const uint64_t b = pb.blk + ((uint64_t)e0 >> 3);
+        const U4 tm = philox4x32_10_v((uint32_t)b, (uint32_t)(b >> 32), kBlockTopM, pb.rot, k0, k1,
+                                      kPhiloxM0, kPhiloxM1);
+        const U4 tw = philox4x32_10_v((uint32_t)b, (uint32_t)(b >> 32), kBlockTopW, pb.rot, k0, k1,
+                                      kPhiloxM0, kPhiloxM1);
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) {
+          zmu_m[j] = fmaf((float)u4_half(tm, j), -1.0f / 65536.0f, C.zoff);
+          zmu_w[j] = fmaf((float)u4_half(tw, j), -1.0f / 65536.0f, C.zoff);
+        }
+      }
+      uint32_t om[kVec], ow[kVec];
+#pragma unroll
+      for (int j = 0; j < kVec; ++j) {
+        const float zm = fmaf(fast_log1p<REG>(fabsf(mm[j])), C.idm, zmu_m[j]);
+        const float fzm = __builtin_amdgcn_fractf(zm);
+        const float cm = __uint_as_float(
+            __float_as_uint(__builtin_amdgcn_fmed3f(zm - fzm, 0.0f, kKM)) |
+            (__float_as_uint(mm[j]) & 0x80000000u));
+        om[j] = __float_as_uint(cm + kCodeBias);
+        // (a negative v counts as 0, as on the exact path; with a NaN among
+        // the v, delta_w is 0 and so is every code)
+        const float s = __builtin_amdgcn_sqrtf(fmaxf(vv[j], 0.0f));
+        const float x = __builtin_amdgcn_fmed3f(fmaf(s, C.wmin, C.we), C.xmin, 1.0f);
+        const float ef = (float)__builtin_amdgcn_frexp_expf(x);
+        const float l2 = __builtin_amdgcn_logf(__builtin_amdgcn_frexp_mantf(x));
+        const float A = ef * C.ch;
+        const float fA = __builtin_amdgcn_fractf(A);
+        const float zw = fmaf(l2, C.cf, fmaf(ef, C.cl, fA + zmu_w[j]));
+        const float fzw = __builtin_amdgcn_fractf(zw);
+        ow[j] = __float_as_uint(
+            __builtin_amdgcn_fmed3f((A - fA) + (zw - fzw), 0.0f, kKW) + kCodeBias);
+        const uint32_t um = unsure(fzm, fmaf(zm, C.hk2, C.hk3));
+        const uint32_t uw = unsure(fzw, fmaf(A, C.nk7, C.hk8));
+        if (j < n) flags |= (um << j) | (uw << (8 + j));
+      }
+      if (n == kVec) {
+        vu4 a, b;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a[i] = pack_lo16(om[2 * i + 1], om[2 * i]);
+          b[i] = pack_lo16(ow[2 * i + 1], ow[2 * i]);
+        }
+        *(vu4u *)(q_m + e0) = a;
+        *(vu4u *)(q_w + e0) = b;
+      } else {
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) {
+          if (j < n) {
+            q_m[e0 + j] = (int16_t)(uint16_t)om[j];
+            q_w[e0 + j] = (int16_t)(uint16_t)ow[j];
+          }
+        }
+      }
+    }
+    // The codes left open join the queues, which hold those of an iteration
+    // (64 lanes x 8) and the at most 63 that the previous one left.
+    if (__ballot(flags != 0)) {
+      const uint32_t fm = flags & 0xFFu, fw = flags >> 8;
+      const uint32_t cnt = (uint32_t)__builtin_popcount(fm) | ((uint32_t)__builtin_popcount(fw) << 16);
+      const uint32_t incl = wave_scan_incl(cnt);
+      const uint32_t excl = incl - cnt, off = (uint32_t)(e0 - beg);
+      uint32_t pos = head_m + len_m + (excl & 0xFFFFu);
+      for (uint32_t f = fm; f != 0u; f &= f - 1u)
+        queue_m[pos++ & (kQuantQueue - 1)] = off + (uint32_t)__builtin_ctz(f);
+      pos = head_w + len_w + (excl >> 16);
+      for (uint32_t f = fw; f != 0u; f &= f - 1u)
+        queue_w[pos++ & (kQuantQueue - 1)] = off + (uint32_t)__builtin_ctz(f);
+      const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+      len_m += tot & 0xFFFFu;
+      len_w += tot >> 16;
+    }
+    // (the exact codes overwrite the fast ones: same wavefront, so the stores
+    // stay in program order)
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    while (len_m >= 64u || (it == n_it && len_m > 0u)) {
+      const uint32_t nb = len_m < 64u ? len_m : 64u;
+      if (lane < nb) {
+        const int64_t i = beg + queue_m[(head_m + lane) & (kQuantQueue - 1)];
+        float a;
+        int lo, hi;
+        exact_quant_m_pair(m[i], G, a, lo, hi);
+        q_m[i] = (int16_t)quant_draw<INJ>(lo, hi, a, G.zm, i, 0, u_m, pb, k0, k1);
+      }
+      head_m += nb;
+      len_m -= nb;
+    }
+    while (len_w >= 64u || (it == n_it && len_w > 0u)) {
+      const uint32_t nb = len_w < 64u ? len_w : 64u;
+      if (lane < nb) {
+        const int64_t i = beg + queue_w[(head_w + lane) & (kQuantQueue - 1)];
+        float a;
+        int lo, hi;
+        exact_quant_w_pair(v[i], G, epsf, a, lo, hi);
+        q_w[i] = (int16_t)quant_draw<INJ>(lo, hi, a, G.zw, i, 1, u_w, pb, k0, k1);
+      }
+      head_w += nb;
+      len_w -= nb;
+    }
+  }
+}
+
+template <bool INJ>
 __global__ __launch_bounds__(kThreads) void quant_kernel(const float *__restrict__ m,
                                                          const float *__restrict__ v, int64_t n,
-                                                         int16_t *__restrict__ q_m,
-                                                         int16_t *__restrict__ q_w,
+                                                         int64_t run, int16_t *q_m, int16_t *q_w,
                                                          const Slot *__restrict__ slot, int par,
                                                          double eps, uint64_t seed,
-                                                         int noise_mode, const float *__restrict__ u_m,
+                                                         const float *__restrict__ u_m,
                                                          const float *__restrict__ u_w) {
-  const Grid G = slot->grid[par];
+  const Grid &G = slot->grid[par];
   const float epsf = (float)eps;
+  const int64_t beg = (int64_t)blockIdx.x * run;
+  const int64_t end = beg + run < n ? beg + run : n;
+  const Bounds B = make_bounds(nullptr, &G, 0.0f, 0.0f);
+  const float hb = INJ ? 0.0f : 0x1p-17f;   // half a bucket of the uniform's top 16 bits
+  QuantConst C;
+  C.idm = G.fast[kIdm];
+  C.hk2 = -B.k2;
+  C.hk3 = 0.5f - (B.k3 + hb);
+  C.cf = G.fast[kNl2dw];
+  C.ch = G.fast[kCwHi];
+  C.cl = G.fast[kCwLo];
+  C.wmin = G.wmin;
+  C.we = G.fast[kWe];
+  C.xmin = G.fast[kXMin];
+  C.nk7 = -B.k7;
+  // v_sqrt_f32 was measured over normal inputs: a subnormal v's root, below
+  // 1.1e-19, is within rounding of nothing beside any eps of 1e-10 or more
+  C.hk8 = epsf >= 1e-10f ? 0.5f - (B.k8 + hb) : -1.0f;
+  C.zoff = 1.0f - hb;
+  __shared__ uint32_t qbuf[kThreads / 64][2 * kQuantQueue];
+  uint32_t *queue = qbuf[threadIdx.x >> 6];
   const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
-  const int64_t beg = (int64_t)blockIdx.x * kChunk;
-  const int64_t end = beg + kChunk < n ? beg + kChunk : n;
-  for (int64_t e0 = beg + (int64_t)threadIdx.x * kVec; e0 < end; e0 += (int64_t)kThreads * kVec) {
-    U4 top_m{}, top_w{}, low{};
-    if (noise_mode == LUMA_NOISE_PHILOX) {
-      top_m = philox_block((uint64_t)e0, PhiloxBase{0, 0}, kBlockTopM, k0, k1);
-      top_w = philox_block((uint64_t)e0, PhiloxBase{0, 0}, kBlockTopW, k0, k1);
-      low = philox_block((uint64_t)e0, PhiloxBase{0, 0}, kBlockLow, k0, k1);
-    }
-    for (int j = 0; j < kVec; ++j) {
-      const int64_t i = e0 + j;
-      if (i >= end) break;
-      float um, uw;
-      if (noise_mode == LUMA_NOISE_PHILOX) {
-        uint32_t bm, bw;
-        philox_uniform_bits(top_m, top_w, low, (uint64_t)i, bm, bw);
-        um = (float)bm * 0x1p-24f;
-        uw = (float)bw * 0x1p-24f;
-      } else {
-        um = u_m[i];
-        uw = u_w[i];
-      }
-      q_m[i] = (int16_t)exact_quant_m(m[i], G, um);
-      q_w[i] = (int16_t)(uint16_t)exact_quant_w(v[i], G, epsf, uw);
-    }
-  }
+  // the log1p form of the largest |m| (the decode side has no part here)
+  const int reg = momentum_regime(0.0f, G.sm);
+  if (reg == kRegSmall)
+    quant_body<INJ, kRegSmall>(m, v, beg, end, q_m, q_w, G, C, epsf, k0, k1, u_m, u_w, queue);
+  else if (reg == kRegMedium)
+    quant_body<INJ, kRegMedium>(m, v, beg, end, q_m, q_w, G, C, epsf, k0, k1, u_m, u_w, queue);
+  else
+    quant_body<INJ, kRegGeneral>(m, v, beg, end, q_m, q_w, G, C, epsf, k0, k1, u_m, u_w, queue);
 }
 
 // Step scalars of steps t0 .. t0+n-1 (luma_hyper_rows).
@@ -2929,16 +3196,24 @@ int luma_quantize(const float *m, const float *v, int64_t numel, int16_t *q_m, i
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t nch = (numel + kChunk - 1) / kChunk;
   if (nch > 0x7fffffff) return fail("luma_quantize: tensor too large");
+  const int64_t nmax = 2 * nch < kMaxBlocks ? 2 * nch : kMaxBlocks;
+  constexpr int64_t kIter = kThreads * kVec;
+  const int64_t run = ((numel + kIter - 1) / kIter + kQuantBlocks - 1) / kQuantBlocks * kIter;
+  const int64_t runs = (numel + run - 1) / run;
   Slot *S = static_cast<Slot *>(slot);
   const int par = (int)(step & 1);
-  hipLaunchKernelGGL(quant_max_kernel, dim3((unsigned)nch), dim3(kThreads), 0, s, m, v, numel,
+  hipLaunchKernelGGL(quant_max_kernel, dim3((unsigned)nmax), dim3(kMaxThreads), 0, s, m, v, numel,
                      partials);
   if (int r = check_launch("luma_quantize: max launch")) return r;
-  hipLaunchKernelGGL(quant_finalize_kernel, dim3(1), dim3(64), 0, s, partials, (int)nch, S, step,
+  hipLaunchKernelGGL(quant_finalize_kernel, dim3(1), dim3(kThreads), 0, s, partials, (int)nmax, S, step,
                      eps);
   if (int r = check_launch("luma_quantize: finalize launch")) return r;
-  hipLaunchKernelGGL(quant_kernel, dim3((unsigned)nch), dim3(kThreads), 0, s, m, v, numel, q_m, q_w,
-                     (const Slot *)S, par, eps, seed, noise_mode, u_m, u_w);
+  if (noise_mode == LUMA_NOISE_INJECTED)
+    hipLaunchKernelGGL(quant_kernel<true>, dim3((unsigned)runs), dim3(kThreads), 0, s, m, v, numel,
+                       run, q_m, q_w, (const Slot *)S, par, eps, seed, u_m, u_w);
+  else
+    hipLaunchKernelGGL(quant_kernel<false>, dim3((unsigned)runs), dim3(kThreads), 0, s, m, v, numel,
+                       run, q_m, q_w, (const Slot *)S, par, eps, seed, u_m, u_w);
   return check_launch("luma_quantize: launch");
 }
 

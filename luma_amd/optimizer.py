@@ -50,6 +50,16 @@ def _is_dense(t: torch.Tensor) -> bool:
             or t.is_contiguous(memory_format=torch.channels_last_3d))
 
 
+def _as_moment(x, param: torch.Tensor) -> torch.Tensor:
+    """x as float32 on the parameter's device in the parameter's layout: x
+    itself where it is that already (the quantise kernels only read it)."""
+    if (type(x) is torch.Tensor and x.dtype == torch.float32 and x.device == param.device
+            and x.shape == param.shape and x.stride() == param.stride() and _is_dense(param)
+            and not x.is_neg()):
+        return x
+    return torch.empty_like(param, dtype=torch.float32).copy_(x)
+
+
 def _ptr(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None else t.data_ptr()
 
@@ -495,7 +505,8 @@ class _Engine:
     def quantize(self, m, v, q_m, q_w, slot, step, eps, seed, noise_mode, u_m, u_w):
         n = m.numel()
         nch = (n + L.CHUNK_ELEMS - 1) // L.CHUNK_ELEMS
-        ws = torch.empty(max(2 * nch, 2), dtype=torch.float32, device=self.device)
+        ws = torch.empty(self.lib.luma_workspace_bytes(max(nch, 1)) // 4, dtype=torch.float32,
+                         device=self.device)
         L.check(self.lib.luma_quantize(m.data_ptr(), v.data_ptr(), n, q_m.data_ptr(),
                                        q_w.data_ptr(), slot.data_ptr(), step, float(eps),
                                        seed & _MASK64, noise_mode, _ptr(u_m), _ptr(u_w),
@@ -822,8 +833,8 @@ class LUMA(Optimizer):
             step = int(step_val.item() if isinstance(step_val, torch.Tensor) else step_val)
             param = self._unwrap_tensor(p)
             engine = self._get_engine(param.device)
-            m = torch.empty_like(param, dtype=torch.float32).copy_(s["exp_avg"])
-            v = torch.empty_like(param, dtype=torch.float32).copy_(s["exp_avg_sq"])
+            m = _as_moment(s["exp_avg"], param)
+            v = _as_moment(s["exp_avg_sq"], param)
             q_m = torch.empty_like(param, dtype=torch.int16)
             q_w = torch.empty_like(param, dtype=torch.int16)
             state = self.state[p]
