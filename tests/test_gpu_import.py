@@ -137,3 +137,28 @@ def test_moments_in_other_layouts():
         codes.append((opt.state[p]["Q_m"], opt.state[p]["Q_w"]))
     for a, b in codes[1:]:
         assert torch.equal(a, codes[0][0]) and torch.equal(b, codes[0][1])
+
+
+# x_top = log1p(S_m) on both sides of 1/8 and of 1/2, and the scale of S_v
+# where exp's argument passes 80 (eps 1e-30)
+@pytest.mark.parametrize("s_m,s_v,eps", [(1e-9, 0.0, 1e-8), (1e-3, 1e-6, 1e-8), (0.133, 1e-4, 1e-8),
+                                         (0.1332, 1e-12, 1e-8), (0.5, 1e-2, 1e-8),
+                                         (0.6485, 1.0, 1e-12), (0.649, 4.0, 1e-8),
+                                         (40.0, 100.0, 1e-8), (0.1, 1e4, 1e-20),
+                                         (0.1, 1e16, 1e-30)])
+@pytest.mark.parametrize("more", [0, 1, 2, 3])
+def test_every_code_decodes_exactly(s_m, s_v, eps, more):
+    print("case", s_m, s_v, eps, more, flush=True)
+    n = (1 << 16) + more
+    codes = (torch.arange(n) & 0xFFFF).to(torch.int32).to(torch.int16)
+    p = torch.nn.Parameter(torch.zeros(n, device=DEV))
+    opt = LUMA([p], eps=eps)
+    sd = opt.state_dict()
+    sd["state"] = {0: {"step": 5, "param_id": 0, "Q_m": codes.to(DEV), "Q_w": codes.to(DEV),
+                       "S_m": s_m, "S_v": s_v}}
+    opt.load_state_dict(sd)
+    out = opt.export_adamw_state()["state"][0]
+    w_min, delta_m, _, delta_w, _ = O.precompute(s_m, s_v, eps)
+    assert torch.equal(out["exp_avg"].cpu(), O.decode_momentum(codes, delta_m, "cr"))
+    assert torch.equal(out["exp_avg_sq"].cpu(),
+                       O.decode_second_moment(codes, w_min, delta_w, eps, "cr"))
