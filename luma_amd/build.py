@@ -36,6 +36,8 @@ FLAGS = [
     "-ffp-contract=off",
     "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # an access that claims more alignment than its pointer has
+    "-Werror=align-mismatch",
     "-I", os.path.join(ROOT, "include"),
 ]
 

@@ -906,13 +906,22 @@ __device__ __forceinline__ float grad_hi(uint32_t w) {
 // the exact path has run for them, some iterations later, and those late
 // 2-byte stores are cheap while the line is still in L2 but cost a
 // partial-line write-back to HBM once it has been evicted.
-template <typename V>
-__device__ __forceinline__ V load_stream(const LUMA_GLOBAL V *p) {
+// They take pointers to the element-aligned vector types by name: a template
+// would deduce the type without its alignment, and so promise the compiler 16
+// bytes (which the build's -Werror=align-mismatch refuses).
+__device__ __forceinline__ vu4 load_stream(const LUMA_GLOBAL vu4u *p) {
   return __builtin_nontemporal_load(p);
 }
 
-template <typename V>
-__device__ __forceinline__ void store_stream(V v, LUMA_GLOBAL V *p) {
+__device__ __forceinline__ vf4 load_stream(const LUMA_GLOBAL vf4u *p) {
+  return __builtin_nontemporal_load(p);
+}
+
+__device__ __forceinline__ void store_stream(vu4 v, LUMA_GLOBAL vu4u *p) {
+  __builtin_nontemporal_store(v, p);
+}
+
+__device__ __forceinline__ void store_stream(vf4 v, LUMA_GLOBAL vf4u *p) {
   __builtin_nontemporal_store(v, p);
 }
 
