@@ -151,7 +151,9 @@ class _Engine:
         self._numel_key = None       # bytes of its numel column and chunk layout (chunk table)
         self._first = None           # first_chunk column of that layout
         self._record = L.CHUNK_ELEMS # chunk length of the uploaded chunk table
-        self._chunk = L.CHUNK_ELEMS  # that of the last launch (its parts, if split)
+        self._chunk = L.CHUNK_ELEMS  # that of its launches (the parts, if split)
+        self._split_flags = 0        # their LUMA_FLAG_SPLIT
+        self._need = 0               # float32 words of their workspace
         self.chunk_elems = 0         # fixed chunk length (a power of two), 0: chunk_for's choice
         self.small_tensors = True    # step tensors of <= SMALL_TENSOR elements a wavefront each
         self._small_chunks = 0       # trailing chunk records of such tensors (uploaded table)
@@ -280,7 +282,7 @@ class _Engine:
         caller has compared them already."""
         capturing = torch.cuda.is_current_stream_capturing()
         n = len(tt)
-        setting = (self.chunk_elems, self._small_limit(), self._medium_limit())
+        setting = (self.chunk_elems, self._small_limit(), self._medium_limit(), self.split)
         same_src = (self._tensor_src is not None and self._tensor_src[0] is tt
                     and self._tensor_src[1] == setting)
         if moved and same_src:
@@ -296,14 +298,11 @@ class _Engine:
                 raise self._capture_error("a param group's hyper-parameters")
             self._d_groups = self._upload(groups)
             self._group_key = gkey
-        self._chunk = self.part(n_chunks - self._small_chunks, self._record)
-        if self._splits():
-            flags |= L.FLAG_SPLIT
-        need = self.lib.luma_workspace_bytes(n_chunks + L.SPLIT_CHUNKS) // 4
-        if self._partials is None or self._partials.numel() < need:
+        flags |= self._split_flags
+        if self._partials is None or self._partials.numel() < self._need:
             if capturing:
                 raise self._capture_error("the chunk count")
-            self._partials = torch.empty(need, dtype=torch.float32, device=self.device)
+            self._partials = torch.empty(self._need, dtype=torch.float32, device=self.device)
         if capturing:
             tables = (self._d_tensors, self._d_chunks, self._d_groups, self._partials)
             if not self._captured or any(x is not y for x, y in zip(self._captured[-1], tables)):
@@ -399,6 +398,11 @@ class _Engine:
         else:
             tt["first_chunk"] = self._first
             key = tt.tobytes()
+        # how its launches are split (here and not on each launch: a step of a
+        # few tensors is host-bound)
+        self._chunk = self.part(self._n_chunks - self._small_chunks, c)
+        self._split_flags = L.FLAG_SPLIT if self._splits() else 0
+        self._need = self.lib.luma_workspace_bytes(self._n_chunks + L.SPLIT_CHUNKS) // 4
         if key != self._tensor_key:
             # the last few uploaded tables stay on the device: a loop whose
             # gradients alternate between buffers re-uses them, no upload

@@ -102,3 +102,23 @@ def test_per_tensor_op_equals_step(n):
         s = opt.state_dict()["state"][0]
         assert torch.equal(s["Q_m"], q_m) and torch.equal(s["Q_w"], q_w), t
         assert F.slot_state(slot) == (s["step"], s["S_m"], s["S_v"]), t
+
+
+def test_planned_steps_take_the_split_of_their_table():
+    """How a set is split is worked out when its table changes or a setting
+    does, not on each step (a step of a few tensors is host-bound)."""
+    oa, ob, step = _pair(SETS["edges"], torch.float32, 34)
+    step(0)
+    step(1)
+    calls = []
+    eng = oa._engine
+    splits = eng._splits
+    eng._splits = lambda: calls.append(1) or splits()
+    for p in oa.param_groups[0]["params"]:
+        p.grad = torch.zeros_like(p)
+    oa.step()                    # a planned step whose gradients moved
+    oa.step()                    # and one where nothing did
+    assert not calls and eng._chunk == 2048
+    eng.split = False
+    oa.step()
+    assert calls and eng._chunk == 16384
