@@ -127,18 +127,25 @@ extern "C" {
 /* luma_step flags. */
 #define LUMA_FLAG_EXACT_ONLY 1 /* take the exact per-element path everywhere */
 /*
- * Let the step give a small set more workgroups than it has chunk records: in
- * a set of at most 2048 workgroup and medium records the medium ones take a
- * workgroup each, and all of them are split into 2^luma_split_shift parts
- * of down to LUMA_CHUNK_ELEMS_MIN elements, which then are the chunks (of the
- * code summaries too).  The results do not depend on it.  `partials` then needs
- * luma_workspace_bytes(n_chunks + LUMA_SPLIT_CHUNKS) (luma_step_tensor: plus
- * LUMA_SPLIT_CHUNKS likewise; luma_step_noalloc's own workspace has the room,
- * and beyond LUMA_NOALLOC_MAX_CHUNKS - LUMA_SPLIT_CHUNKS chunks it ignores
- * the flag).  Without the flag every record is one chunk.
+ * Let the step give a small set more workgroups than it has chunk records:
+ * the medium records take a workgroup each where luma_split_plan says so, and
+ * the workgroup records (those medium ones among them) are split into
+ * 2^(its value) parts of down to LUMA_CHUNK_ELEMS_MIN elements, which then are
+ * the chunks (of the code summaries too).  The results do not depend on it.
+ * `partials` then needs luma_workspace_bytes(n_chunks + LUMA_SPLIT_CHUNKS)
+ * (luma_step_tensor: plus LUMA_SPLIT_CHUNKS likewise; luma_step_noalloc's own
+ * workspace has the room, and beyond LUMA_NOALLOC_MAX_CHUNKS -
+ * LUMA_SPLIT_CHUNKS chunks it ignores the flag).  Without the flag every
+ * record is one chunk.
  */
 #define LUMA_FLAG_SPLIT 2
 #define LUMA_SPLIT_CHUNKS 1024
+/*
+ * For LUMA_FLAG_SPLIT, in luma_step's flags: the elements of the longest medium
+ * tensor, which luma_split_plan's rule takes (absent: LUMA_MEDIUM_TENSOR).
+ */
+#define LUMA_FLAG_LONGEST_SHIFT 8
+#define LUMA_FLAG_LONGEST(elems) ((int32_t)(elems) << LUMA_FLAG_LONGEST_SHIFT)
 
 /* One parameter tensor taking part in a step. */
 typedef struct LumaTensor {
@@ -223,7 +230,8 @@ typedef struct LumaStepArgs {
                                 others (8 elements per lane and iteration); meant for
                                 tensors of at most LUMA_MEDIUM_TENSOR elements, one
                                 chunk each (any chunk is stepped correctly).  Such
-                                tensors keep no code summaries.  0: none */
+                                tensors keep no code summaries.  LUMA_FLAG_SPLIT may
+                                give them a workgroup each instead.  0: none */
   int32_t reserved;          /* 0 */
   LumaScaling scaling;       /* both NULL: unscaled gradients, always step */
 } LumaStepArgs;
@@ -250,9 +258,17 @@ void luma_layout(int32_t out[8]);
 size_t luma_workspace_bytes(int32_t n_chunks);
 
 /*
- * How far LUMA_FLAG_SPLIT splits `records` workgroup and medium records of
- * chunk_elems elements (luma_step: n_chunks - small_chunks): log2 of the parts.
+ * How LUMA_FLAG_SPLIT shares out a launch of `records` workgroup records of
+ * chunk_elems elements (luma_step: n_chunks - medium_chunks - small_chunks),
+ * `medium` and `small` records (medium_chunks, small_chunks), the longest
+ * medium tensor of `medium_longest` elements (0: LUMA_MEDIUM_TENSOR): returns
+ * log2 of the parts of a workgroup record; *wide (may be NULL) is 1 where the
+ * medium records take a workgroup each, which then are split too.
  */
+int32_t luma_split_plan(int32_t records, int32_t medium, int32_t small, int32_t medium_longest,
+                        int32_t chunk_elems, int32_t *wide);
+
+/* luma_split_plan of `records` workgroup records alone. */
 int32_t luma_split_shift(int32_t records, int32_t chunk_elems);
 
 /* Summary words a tensor of numel elements needs for chunks of chunk_elems elements. */

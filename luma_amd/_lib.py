@@ -30,6 +30,7 @@ GRAD_F32, GRAD_BF16, GRAD_F16 = 0, 1, 2
 NOISE_PHILOX, NOISE_INJECTED = 0, 1
 FLAG_EXACT_ONLY = 1
 FLAG_SPLIT = 2               # LUMA_FLAG_SPLIT
+FLAG_LONGEST_SHIFT = 8       # LUMA_FLAG_LONGEST(elems): elems << this
 SPLIT_CHUNKS = 1024          # LUMA_SPLIT_CHUNKS: workspace chunks it may add
 
 TENSOR_DTYPE = np.dtype([
@@ -87,6 +88,7 @@ _SIGNATURES = {
     "luma_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int32]),
     "luma_summary_words": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int32]),
     "luma_split_shift": (ctypes.c_int32, [ctypes.c_int32, ctypes.c_int32]),
+    "luma_split_plan": (ctypes.c_int32, [ctypes.c_int32] * 5 + [ctypes.POINTER(ctypes.c_int32)]),
     "luma_layout": (None, [ctypes.POINTER(ctypes.c_int32)]),
     "luma_step": (ctypes.c_int, [ctypes.POINTER(StepArgs), _VP]),
     "luma_step_noalloc": (ctypes.c_int, [ctypes.POINTER(StepArgs), _VP]),

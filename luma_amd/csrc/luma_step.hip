@@ -113,7 +113,7 @@ static_assert(sizeof(Tensor) == sizeof(LumaTensor), "tensor layout");
 // wavefront-per-tensor exact kernels (small tensors).
 //
 // A launch may split every workgroup record into 2^split parts of 2^wg_shift
-// elements, a workgroup each (split_records): the part is then the chunk that
+// elements, a workgroup each (luma_split_plan): the part is then the chunk that
 // the kernels work on, and parts past the tensor's end have no workgroup's
 // work.  Wavefront records are never split.  part_record numbers the parts
 // and the wavefront records in one row: their places in `partials`.
@@ -3036,35 +3036,84 @@ int64_t luma_summary_words(int64_t numel, int32_t chunk_elems) {
   return ((numel - 1) / chunk_elems + 1) * LUMA_SUMMARY_WORDS;
 }
 
-// A launch of about as many workgroups as the chip holds at once (768: three
-// to a CU, pass 2's registers) is as long as one workgroup, and a workgroup
-// as long as its iterations of 2,048 elements (about 2 us each in pass 2,
-// after 10 us of set-up and fallback): more and shorter parts are then free.
-// Parts of 8,192 elements while there are at most 1,024 of them, of 4,096 at
-// most 768, of 2,048 at most 384 (with more, pass 1 and finalize lose what
-// pass 2 gains).  Step times (us) by the part's length, 16,384 / 8,192 /
+// LUMA_FLAG_SPLIT's two rules.  A launch of about as many workgroups as the
+// chip holds at once (768: three to a CU, pass 2's registers) is as long as one
+// workgroup, and a workgroup as long as its iterations of 2,048 elements
+// (about 2 us each in pass 2, after 10 us of set-up and fallback).  All times
+// here are steps in us, graph replays.
+//
+// Medium tensors in a workgroup each (wide) or in a wavefront each.  One
+// wavefront takes 3.4 us per 512 elements and, beside workgroup records, starts
+// after them: the launch ends on the longest medium tensor.  A workgroup is
+// four times faster and takes four times the slots.  Wavefronts -> wide, by
+// the tensors' elements (and workgroup records, split as below in either form):
+//                               257-512       1,025-2,048    4,097-8,192
+//   100                       26.2 -> 22.1   33.2 -> 22.7   66.8 -> 29.4
+//   500                       22.9 -> 23.1   31.7 -> 28.2   77.3 -> 42.4
+//   700                       23.8 -> 25.7   33.7 -> 32.5   81.2 -> 52.6
+//   1,200                     30.7 -> 40.6   41.3 -> 48.3   95.1 -> 88.1
+//   2,000                     29.9 -> 51.3   44.8 -> 65.8  110.1 -> 126.7
+//   30, 100 records           31.1 -> 32.0   34.5 -> 31.7   73.2 -> 33.8
+//   100, 100 records          31.2 -> 35.6   35.2 -> 34.7   75.1 -> 42.1
+//   300, 300 records          51.2 -> 57.5   53.5 -> 58.5   91.6 -> 62.6
+//   300, 800 records          96.7 -> 97.3   97.2 -> 100.2 134.2 -> 105.1
+//   1,000, 800 records        99.2 -> 101.4 104.8 -> 107.6 154.0 -> 136.4
+// So the tensors may be as many as their length pays for: alone (with small
+// tensors' workgroups beside them) 448 and one more per 10 elements of the
+// longest, beside records one per 8.
+//
+// Splitting the workgroup records: more and shorter parts are free as long as
+// the workgroups are one round: parts of 8,192 elements while there are at
+// most 816, of 4,096 at most 768, of 2,048 at most 384 (with more, pass 1 and
+// finalize lose what pass 2 gains).  By the part's length, 16,384 / 8,192 /
 // 4,096 / 2,048 elements:
-//   1 tensor of 200,000 (13 records)       37.9  28.7  25.3  25.4
-//   1 tensor of 1,000,003 (62)             39.0  29.3  26.1  27.9
-//   3 tensors, 2.2M elements (138)         42.5  39.7  36.6  45.2
-//   1 tensor of 4,185,079 (256)            45.4  44.5  46.2
-//   400 tensors, 4.1M elements (393)       60.9  53.7  57.5  69.4
-//   1 tensor of 12,500,000 (763)           82.3  90.0 109.0
-int32_t luma_split_shift(int32_t records, int32_t chunk_elems) {
-  if (records <= 0 || chunk_elems <= 0) return 0;
+//   50 records                  40.0  31.0  26.4  26.3
+//   100 records                 44.2  34.0  31.1  30.3
+//   200 records                 45.5  41.8  40.0
+//   340 records                 59.4  52.3  56.7
+//   400 records                 60.3  59.9
+//   500 records                 62.7  66.9
+// Medium tensors' wavefronts come after the parts; where they are long, only
+// parts that leave them CUs of their own (256) are worth it: 100 records and
+// 100 tensors of 1,025-2,048 elements 42.0, 34.0, 36.8, 43.2.
+// A wide medium tensor fills one part or a few of its record's; workgroups go
+// to the eight XCDs in turn, so the others lie idle: its tensors' first parts
+// have the 256 >> split CUs of every second, fourth or eighth XCD's turn.
+// Beyond 204, 120 and 51 of them that costs more than it gains: 500 tensors of
+// 257-512 elements 23.1, split 32.4; beside 5 records 100 of 1,025-2,048
+// elements 36.4, 31.0, 27.8, 36.7 by the part's length, 200 36.9, 31.8, 37.0.
+int32_t luma_split_plan(int32_t records, int32_t medium, int32_t small, int32_t longest,
+                        int32_t chunk_elems, int32_t *wide) {
+  if (wide) *wide = 0;
+  if (records < 0 || medium < 0 || small < 0 || chunk_elems <= 0) return 0;
+  constexpr int64_t kMost = 2048;   // records of the largest set that the first rule was measured on
+  const int64_t r = records, m = medium;
+  if (longest <= 0) longest = LUMA_MEDIUM_TENSOR;
+  const bool w = m > 0 && r + m <= kMost &&
+                 (r == 0 ? m + small / 4 <= 448 + longest / 10 : m <= longest / 8);
+  if (wide) *wide = w ? 1 : 0;
+  if (r == 0 && !w) return 0;
   const int32_t shift = 31 - __builtin_clz((unsigned)chunk_elems);
   const auto fits = [&](int32_t split) -> bool {
     const int32_t part = shift - split;
-    const int64_t most = part >= 13   ? LUMA_SPLIT_CHUNKS
-                         : part == 12 ? LUMA_SPLIT_CHUNKS * 3 / 4
-                         : part == 11 ? LUMA_SPLIT_CHUNKS * 3 / 8
-                                      : 0;
-    return (int64_t)records << split <= most;
+    if (w) {
+      if (m > (split == 2 ? 120 : 408 >> split)) return false;
+    } else if (m > 0 && longest > 1024 && part < 13) {
+      return (r << split) + (m + 3) / 4 <= (part >= 11 ? 256 : 0);
+    }
+    const int64_t blocks = w ? (r + m) << split : (r << split) + (m + 3) / 4;
+    const int64_t most = part >= 13 ? 816 : part == 12 ? 768 : part == 11 ? 384 : 0;
+    return blocks <= most;
   };
   static_assert(LUMA_CHUNK_ELEMS_MIN == 1 << 11, "shortest part");
+  static_assert(816 <= LUMA_SPLIT_CHUNKS, "the workspace's room for parts");
   int32_t split = 0;
   while (fits(split + 1)) ++split;
   return split;
+}
+
+int32_t luma_split_shift(int32_t records, int32_t chunk_elems) {
+  return records > 0 ? luma_split_plan(records, 0, 0, 0, chunk_elems, nullptr) : 0;
 }
 
 size_t luma_workspace_bytes(int32_t n_chunks) {
@@ -3149,15 +3198,6 @@ static int launch_step(StepSrc src, int32_t n_tensors, int32_t n_chunks, float *
   return mark(3);
 }
 
-// LUMA_FLAG_SPLIT: with at most this many workgroup and medium records, a
-// medium tensor takes a workgroup as the others do.  The wavefront route saves
-// a full chip's workgroup slots (20,000 tensors: pass 2 0.643 -> 0.616 ms with
-// it); on a chip that has slots to spare, one wavefront is only four times
-// slower than four (6 tensors, 11,441 elements: step 58.9 us by wavefronts,
-// 28.8 us by workgroups; 400 tensors, 588 records: 79.7 and 63.3 us; 2,000
-// tensors, 2,396 records: 134.7 and 132.1 us).
-constexpr int32_t kWideRecords = 2048;
-
 static int step_impl(const LumaStepArgs *a, void *stream, void *const *events) {
   if (!a) return fail("luma_step: null args");
   if (a->n_tensors <= 0 || a->n_chunks <= 0) return 0;
@@ -3180,10 +3220,11 @@ static int step_impl(const LumaStepArgs *a, void *stream, void *const *events) {
   src.small_from = a->n_chunks - a->small_chunks;
   src.medium_from = src.small_from - a->medium_chunks;
   src.n_chunks = a->n_chunks;
-  if ((a->flags & LUMA_FLAG_SPLIT) != 0 && (a->flags & LUMA_FLAG_EXACT_ONLY) == 0 &&
-      src.small_from <= kWideRecords) {
-    src.medium_from = src.small_from;   // medium tensors: a workgroup each
-    src.split = luma_split_shift(src.small_from, c);
+  if ((a->flags & LUMA_FLAG_SPLIT) != 0 && (a->flags & LUMA_FLAG_EXACT_ONLY) == 0) {
+    int32_t wide;
+    src.split = luma_split_plan(src.medium_from, a->medium_chunks, a->small_chunks,
+                                a->flags >> LUMA_FLAG_LONGEST_SHIFT, c, &wide);
+    if (wide) src.medium_from = src.small_from;   // medium tensors: a workgroup each
   }
   return launch_step(src, a->n_tensors, a->n_chunks, a->partials, a->base_seed, a->noise_mode,
                      a->flags, static_cast<hipStream_t>(stream), events);

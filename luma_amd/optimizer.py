@@ -160,6 +160,8 @@ class _Engine:
         self.medium_tensors = True   # step tensors of <= MEDIUM_TENSOR elements one wavefront
                                      # each (inside the fast kernels' launches)
         self._medium_chunks = 0      # the records of such tensors, before the small ones
+        self._medium_longest = 0     # elements of the longest of them
+        self._wide = False           # its launches give them a workgroup each
         self.split = True            # let the library split the records of a small set
         self._d_tensors = None
         self._table_cache = {}       # tensor-table bytes -> device copy (most recent last)
@@ -226,17 +228,26 @@ class _Engine:
         return (self.split and not self.chunk_elems
                 and (self._small_limit(), self._medium_limit()) == _ROUTES)
 
-    def part(self, records: int, c: int) -> int:
-        """Length of the chunks that a launch of ``records`` workgroup and
-        medium records of c elements works on."""
-        return c >> self.lib.luma_split_shift(records, c) if self._splits() else c
+    def _split_plan(self, records: int, medium: int, small: int, longest: int,
+                    c: int) -> Tuple[int, bool]:
+        """How a launch of these workgroup, medium and small records (the
+        longest medium tensor of ``longest`` elements) at chunk length c is
+        shared out: the length of its chunks, and whether the medium records
+        take a workgroup each."""
+        if not self._splits():
+            return c, False
+        wide = ctypes.c_int32()
+        shift = self.lib.luma_split_plan(records, medium, small, longest, c, ctypes.byref(wide))
+        return c >> shift, bool(wide.value)
 
     def summary_chunk(self, numels: np.ndarray) -> int:
         """Chunk length that a step over tensors of these sizes keeps code
         summaries for."""
         c = self.chunk_for(numels)
-        big = numels[numels > self._small_limit()]
-        return self.part(int(((big + c - 1) // c).sum()), c)
+        small, medium = self._route_masks(numels, c)
+        big = numels[~small & ~medium]
+        return self._split_plan(int(((big + c - 1) // c).sum()), int(medium.sum()),
+                                int(small.sum()), int(numels[medium].max(initial=0)), c)[0]
 
     def table(self, rows) -> np.ndarray:
         """Tensor table of rows: (param, grad, q_m, q_w, u_m, u_w, slot, param_id,
@@ -334,6 +345,12 @@ class _Engine:
         """Largest tensor stepped by a single wavefront, either route."""
         return max(self._small_limit(), self._medium_limit())
 
+    def _route_masks(self, numels: np.ndarray, c: int):
+        """Which tensors of these sizes are small ones and which medium ones
+        at chunk length c (masks; chunk_layout's runs)."""
+        small = numels <= self._small_limit()
+        return small, ~small & (numels <= min(self._medium_limit(), c))
+
     def chunk_layout(self, numels: np.ndarray, c: int):
         """Chunk table layout of tensors of these sizes at chunk length c: the
         first chunk of every tensor, the chunk records (tensor, index), and
@@ -392,6 +409,8 @@ class _Engine:
             self._n_chunks = len(ch)
             self._small_chunks = n_small
             self._medium_chunks = n_medium
+            self._medium_longest = int(
+                numels[self._route_masks(numels, c)[1]].max(initial=0))
             self._record = c
             self._numel_key = nkey
             self._first = first
@@ -400,8 +419,11 @@ class _Engine:
             key = tt.tobytes()
         # how its launches are split (here and not on each launch: a step of a
         # few tensors is host-bound)
-        self._chunk = self.part(self._n_chunks - self._small_chunks, c)
-        self._split_flags = L.FLAG_SPLIT if self._splits() else 0
+        self._chunk, self._wide = self._split_plan(
+            self._n_chunks - self._small_chunks - self._medium_chunks, self._medium_chunks,
+            self._small_chunks, self._medium_longest, c)
+        self._split_flags = (L.FLAG_SPLIT | self._medium_longest << L.FLAG_LONGEST_SHIFT
+                             if self._splits() else 0)
         self._need = self.lib.luma_workspace_bytes(self._n_chunks + L.SPLIT_CHUNKS) // 4
         if key != self._tensor_key:
             # the last few uploaded tables stay on the device: a loop whose

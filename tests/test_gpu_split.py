@@ -1,7 +1,7 @@
 """LUMA_FLAG_SPLIT: records of a small set split into parts, and its medium
-tensors a workgroup each.  The parts change which threads step an element and
-nothing else, so a split launch equals the unsplit one bit for bit; the
-unsplit routes (one wavefront per medium tensor among them) are compared
+tensors in a workgroup each or in wavefronts beside the parts.  The parts
+change which threads step an element and nothing else, so a split launch
+equals the unsplit one bit for bit; the unsplit routes (one wavefront per medium tensor among them) are compared
 with the oracle here, the split ones by every other parity test."""
 
 import pytest
@@ -24,6 +24,23 @@ SETS = {
     "parts of 4096": [700001, 300, 90000],
     "parts of 8192": [5000003, 12000, 100],
     "many": [300 + 37 * i for i in range(250)] + [16385] * 30 + [9] * 100,
+    "wide, parts of 8192": [20000] * 60 + [300 + 52 * i for i in range(150)],
+    "medium wavefronts beside parts": [16385] * 60 + [300 + i for i in range(150)] + [9] * 30,
+    "medium only, wide and split": [257 + 80 * i for i in range(99)],
+    "medium only, wavefronts": [257 + i % 256 for i in range(701)],
+}
+# the part length, and whether the medium tensors take a workgroup each
+PLANS = {
+    "one element": (16384, False),
+    "edges": (2048, True),
+    "small only": (16384, False),
+    "parts of 4096": (4096, True),
+    "parts of 8192": (8192, False),
+    "many": (16384, True),
+    "wide, parts of 8192": (8192, True),
+    "medium wavefronts beside parts": (4096, False),
+    "medium only, wide and split": (4096, True),
+    "medium only, wavefronts": (16384, False),
 }
 
 
@@ -60,6 +77,8 @@ def test_split_equals_unsplit(name, dtype):
     ob._get_engine(next(iter(ob.param_groups[0]["params"])).device).split = False
     for t in range(4):
         step(t)
+    assert (oa._engine._chunk, oa._engine._wide) == PLANS[name]
+    assert (ob._engine._chunk, ob._engine._wide) == (16384, False)
 
 
 def test_split_changes_between_steps():
