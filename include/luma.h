@@ -57,7 +57,7 @@
 extern "C" {
 #endif
 
-#define LUMA_ABI_VERSION 9
+#define LUMA_ABI_VERSION 10
 
 /*
  * Elements per chunk-table entry (one workgroup's share of a tensor): the

@@ -24,7 +24,7 @@ STEP_TENSOR_CHUNK_MIN = 16384  # LUMA_STEP_TENSOR_CHUNK_MIN
 SLOT_BYTES = 512             # LUMA_SLOT_BYTES
 NOALLOC_MAX_CHUNKS = 262144  # LUMA_NOALLOC_MAX_CHUNKS
 SUMMARY_WORDS = 256          # LUMA_SUMMARY_WORDS (per chunk)
-ABI_VERSION = 9              # LUMA_ABI_VERSION
+ABI_VERSION = 10             # LUMA_ABI_VERSION
 
 GRAD_F32, GRAD_BF16, GRAD_F16 = 0, 1, 2
 NOISE_PHILOX, NOISE_INJECTED = 0, 1
@@ -119,12 +119,14 @@ def load(path: str = LIB_PATH):
             f"{LIB_NAME} not found at {path}; build it with "
             "`python -c 'import luma_amd.build as b; b.build()'` (needs hipcc)")
     lib = ctypes.CDLL(path)
+    # (the version first: a library of another one may lack entry points)
+    lib.luma_abi_version.restype, lib.luma_abi_version.argtypes = _SIGNATURES["luma_abi_version"]
+    if lib.luma_abi_version() != ABI_VERSION:
+        raise LumaLibraryError(f"{LIB_NAME} ABI {lib.luma_abi_version()} != {ABI_VERSION}")
     for name, (res, args) in _SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    if lib.luma_abi_version() != ABI_VERSION:
-        raise LumaLibraryError(f"{LIB_NAME} ABI {lib.luma_abi_version()} != {ABI_VERSION}")
     check_layout(lib)
     _lib = lib
     return lib

@@ -3,6 +3,7 @@
 import ctypes
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -33,6 +34,18 @@ def _declared_symbols():
     text = open(os.path.join(ROOT, "include", "luma.h")).read()
     text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
     return sorted(set(re.findall(r"\b(luma_\w+)\s*\(", text)))
+
+
+def test_library_of_another_abi_is_named(tmp_path, monkeypatch):
+    """A library built from another version of the header, which may lack
+    entry points, is refused by its version."""
+    src = tmp_path / "old.c"
+    src.write_text(f"int luma_abi_version(void) {{ return {L.ABI_VERSION - 1}; }}\n")
+    lib = tmp_path / "libold.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    monkeypatch.setattr(L, "_lib", None)
+    with pytest.raises(L.LumaLibraryError, match=f"ABI {L.ABI_VERSION - 1} != {L.ABI_VERSION}"):
+        L.load(str(lib))
 
 
 def test_library_exports_every_declared_symbol():
