@@ -101,12 +101,6 @@ __device__ __forceinline__ void make_grid_w(double S_v, double eps, Grid &g) {
   g.dwpos = delta_w > 0.0 ? 1 : 0;
 }
 
-__device__ inline void make_grid(double S_m, double S_v, double eps, Grid &g) {
-  make_grid_m(S_m, g);
-  make_grid_w(S_v, eps, g);
-  for (int i = 0; i < 20; ++i) g.fast[i] = 0.0f;
-}
-
 // Decode (functional.py:113-116): m = sgn(q) * expm1(|q| * dm).
 __device__ __forceinline__ float exact_decode_m(int q, float dm) {
   const float e = cr_expm1((float)(q < 0 ? -q : q) * dm);

@@ -46,7 +46,7 @@ constexpr float kSmall = 0.125f;  // polynomial regime bound of expm1 / log1p
 constexpr float kSafety = 2.0f;     // pass 1
 constexpr float kSafety2 = 1.05f;   // pass 2
 
-// Indices into Grid::fast, filled by make_fast (finalize) for the new grid.
+// Indices into Grid::fast, filled by make_fast_m and make_fast_w for the new grid.
 enum FastSlot {
   kIdm = 0,     // f32(1 / dm)
   kYTopM,       // exact y of |m| = S_m (largest momentum bin index)
@@ -269,12 +269,6 @@ __device__ __forceinline__ void make_fast_w(Grid &g, float eps) {
   }
   g.fast[kWe] = (float)((double)g.wmin * (double)eps);
   g.fast[kXMin] = (float)((double)g.wmin / (double)g.wmax);
-}
-
-__device__ inline void make_fast(Grid &g, float eps) {
-  for (int i = 0; i < 20; ++i) g.fast[i] = 0.0f;
-  make_fast_m(g);
-  make_fast_w(g, eps);
 }
 
 // Error bounds of one tensor's fast path for one step (built per workgroup).
