@@ -55,7 +55,7 @@ def _as_moment(x, param: torch.Tensor) -> torch.Tensor:
     itself where it is that already (the quantise kernels only read it)."""
     if (type(x) is torch.Tensor and x.dtype == torch.float32 and x.device == param.device
             and x.shape == param.shape and x.stride() == param.stride() and _is_dense(param)
-            and not x.is_neg()):
+            and not x.is_neg() and not x._is_zerotensor()):
         return x
     return torch.empty_like(param, dtype=torch.float32).copy_(x)
 

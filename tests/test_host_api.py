@@ -36,6 +36,18 @@ def _declared_symbols():
     return sorted(set(re.findall(r"\b(luma_\w+)\s*\(", text)))
 
 
+def test_moments_without_storage_are_converted():
+    """A zero tensor that autograd hands out has no memory to read in place."""
+    from luma_amd.optimizer import _as_moment
+    param = torch.ones(3, 4)
+    zero = torch._efficientzerotensor((3, 4))
+    m = _as_moment(zero, param)
+    assert m.data_ptr() != 0 and torch.equal(m, torch.zeros(3, 4))
+    x = torch.ones(3, 4)
+    assert _as_moment(x, param) is x
+    assert _as_moment(x.double(), param).dtype == torch.float32
+
+
 def test_library_of_another_abi_is_named(tmp_path, monkeypatch):
     """A library built from another version of the header, which may lack
     entry points, is refused by its version."""
