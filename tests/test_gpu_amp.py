@@ -27,8 +27,9 @@ class _Classic(LUMA):
 
 
 def _model():
-    # weights of 8192 (a workgroup per chunk), 3072 (one wavefront each: the
-    # medium route) and 24 elements (the small-tensor kernels), and biases
+    # weights of 8192 and 3072 (medium tensors: a workgroup each, or without
+    # `split` one wavefront each) and of 24 elements (the small-tensor
+    # kernels), and biases
     torch.manual_seed(0)
     return nn.Sequential(nn.Linear(64, 128), nn.GELU(), nn.Linear(128, 24), nn.GELU(),
                          nn.Linear(24, 1)).to(DEV)
@@ -41,12 +42,14 @@ def _state(opt, model):
              for _, s in sorted(sd.items())])
 
 
+@pytest.mark.parametrize("split", [True, False])
 @pytest.mark.parametrize("autocast_dtype", [torch.float16, torch.bfloat16])
-def test_gradscaler_in_kernel_unscale_equals_classic_path(autocast_dtype):
+def test_gradscaler_in_kernel_unscale_equals_classic_path(autocast_dtype, split):
     ma, mb = _model(), _model()
     oa = LUMA(ma.parameters(), lr=1e-3, weight_decay=0.05)
     ob = _Classic(mb.parameters(), lr=1e-3, weight_decay=0.05)
     ob._base_seed = oa._base_seed
+    oa._get_engine(torch.device(DEV, 0)).split = split
     sa = torch.amp.GradScaler("cuda", init_scale=2.0 ** 14, growth_interval=3)
     sb = torch.amp.GradScaler("cuda", init_scale=2.0 ** 14, growth_interval=3)
     gen = torch.Generator(device=DEV).manual_seed(1)
@@ -72,6 +75,7 @@ def test_gradscaler_in_kernel_unscale_equals_classic_path(autocast_dtype):
             assert torch.equal(s1[0], s2[0]) and torch.equal(s1[1], s2[1]), f"step {step}: codes {i}"
             assert s1[2:] == s2[2:], f"step {step}: scales/step {i}: {s1[2:]} vs {s2[2:]}"
     assert qa[0][4] < 12   # the overflow step (and any other) did not count
+    assert oa._engine._medium_chunks == 2 and oa._engine._wide == split
 
 
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16, torch.float16])

@@ -8,6 +8,10 @@ pass 2 through the fast kernel's wavefront route).  Their results must be the
 oracle's, as the workgroup kernels' are, whichever route a tensor takes from
 step to step; a large tensor routed there is stepped correctly too, and the
 code summaries of such a step are not used by the next one.
+
+In small sets the library gives medium tensors a workgroup each
+(LUMA_FLAG_SPLIT, the engine's `split`), so the tests of their wavefront
+route switch that off and check the route taken (`_wide`).
 """
 
 import pytest
@@ -102,11 +106,13 @@ MEDIUM = [513, 600, 1000, 2047, 2048, 2049, 3000, 4095, 4096, 4097, 8191, 8192, 
           70000, 9000]
 
 
+@pytest.mark.parametrize("split", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-def test_medium_tensors_match_oracle(dtype):
+def test_medium_tensors_match_oracle(dtype, split):
     gen = torch.Generator(device=DEV).manual_seed(21)
     params = [(torch.randn(n, device=DEV, generator=gen) * 0.02) for n in MEDIUM]
     pair = SampledPair(params, range(len(MEDIUM)))
+    pair.opt._get_engine(params[0].device).split = split
     for t in range(1, 5):
         g = torch.Generator(device=DEV).manual_seed(700 + t)
         gd = [normal_grad(p.shape, 1e-3, g, DEV, dtype, outliers=1e-2, zeros=0.02)
@@ -115,6 +121,7 @@ def test_medium_tensors_match_oracle(dtype):
         pair.check()
         eng = pair.opt._engine
         assert eng._medium_chunks == sum(1 for n in MEDIUM if L.SMALL_TENSOR < n <= L.MEDIUM_TENSOR)
+        assert eng._wide == split
         assert eng._small_chunks == sum(1 for n in MEDIUM if n <= L.SMALL_TENSOR)
 
 
@@ -133,6 +140,7 @@ def test_medium_route_matches_workgroup_route(scaled):
         p.grad_dtype = None        # allow bf16 gradients on fp32 parameters
     oa, ob = LUMA(a, lr=1e-3, weight_decay=0.01), LUMA(b, lr=1e-3, weight_decay=0.01)
     ob._base_seed = oa._base_seed
+    oa._get_engine(a[0].device).split = False
     ob._get_engine(b[0].device).medium_tensors = False
     scale = 2.0 ** 12
     if scaled:
@@ -151,6 +159,7 @@ def test_medium_route_matches_workgroup_route(scaled):
     torch.cuda.synchronize()
     n_med = sum(1 for n in sizes if L.SMALL_TENSOR < n <= L.MEDIUM_TENSOR)
     assert oa._engine._medium_chunks == n_med and ob._engine._medium_chunks == 0
+    assert not oa._engine._wide
     sa, sb = oa.state_dict()["state"], ob.state_dict()["state"]
     for i, (p, q) in enumerate(zip(a, b)):
         assert torch.equal(sa[i]["Q_m"], sb[i]["Q_m"]), i
@@ -181,10 +190,11 @@ def test_medium_route_for_every_tensor(monkeypatch):
     assert eng._medium_chunks > 0
 
 
-def test_fast_launches_equal_exact_launches_on_every_route():
+@pytest.mark.parametrize("split", [False, True])
+def test_fast_launches_equal_exact_launches_on_every_route(split):
     """A set with small, medium and workgroup tensors: the fast launches (the
     small tensors' pass 1 inside the pass-1 launch, each medium tensor one
-    wavefront) and the exact-only launches (the small tensors' pass 1 in a
+    wavefront, or with split one workgroup) and the exact-only launches (the small tensors' pass 1 in a
     kernel of its own) give the same codes and scales, and parameters within
     1e-6 of their scale (the fast update's bound)."""
     from luma_amd import LUMA
@@ -196,6 +206,7 @@ def test_fast_launches_equal_exact_launches_on_every_route():
     oa, ob = LUMA(a, lr=1e-3), LUMA(b, lr=1e-3)
     ob._base_seed = oa._base_seed
     ob._flags = L.FLAG_EXACT_ONLY
+    oa._get_engine(a[0].device).split = split
     for t in range(4):
         for p, q in zip(a, b):
             g = torch.randn(p.shape, device=DEV, generator=gen) * 1e-3
@@ -204,6 +215,7 @@ def test_fast_launches_equal_exact_launches_on_every_route():
         ob.step()
     torch.cuda.synchronize()
     ea = oa._engine
+    assert ea._wide == split
     assert ea._small_chunks == 3 * sum(1 for n in set(sizes) if n <= L.SMALL_TENSOR)
     assert ea._medium_chunks == 3 * sum(1 for n in set(sizes)
                                         if L.SMALL_TENSOR < n <= L.MEDIUM_TENSOR)
