@@ -1,8 +1,10 @@
 """import_adamw_state takes its codes from the certified fast encode and the
 exact path; they are the oracle's codes bit for bit: around a lane's group,
-the quantise pass's and the max pass's workgroups, in each log1p form, with
-injected and Philox uniforms, and for values that only the exact path takes.
-export_adamw_state decodes every code as the oracle does, at every remainder."""
+the quantise pass's and the max pass's workgroups, over several iterations of
+a workgroup and round its queues, in each log1p form, with injected and
+Philox uniforms, and for values that only the exact path takes.
+export_adamw_state decodes every code as the oracle does, at every remainder
+and past a workgroup's first iteration."""
 
 import numpy as np
 import pytest
@@ -43,13 +45,14 @@ def _uniforms(n, seed):
                  for i in (0, 1))
 
 
-def _check(m, v, inject, eps=EPS):
+def _check(m, v, inject, eps=EPS, u=None):
     n = m.numel()
     p = torch.nn.Parameter(torch.zeros(n, device=DEV))
     opt = LUMA([p], eps=eps)
     opt._base_seed = 12345
     if inject:
-        u = tuple(torch.rand(n, generator=torch.Generator().manual_seed(n + i)) for i in (1, 2))
+        if u is None:
+            u = tuple(torch.rand(n, generator=torch.Generator().manual_seed(n + i)) for i in (1, 2))
         opt.inject_noise({p: tuple(x.to(DEV) for x in u)})
     else:
         u = _uniforms(n, make_step_seed(opt._base_seed, 0, 0))
@@ -78,6 +81,40 @@ def _moments(n, scale):
 def test_codes_at_edges(n, inject):
     print("case", n, inject, flush=True)
     _check(*_moments(n, 1e-3), inject)
+
+
+# the quantise pass gives each of 1,024 workgroups more than one iteration of
+# 2,048 elements above 2,097,152: two (the last workgroup's run of one
+# element), three, and six with ragged ends
+LARGE = [(1 << 21) + 1, (2 << 21) + 2049, 10500003]
+
+
+@pytest.mark.parametrize("inject", [False, True])
+@pytest.mark.parametrize("n", LARGE)
+def test_codes_over_several_iterations(n, inject):
+    print("case", n, inject, flush=True)
+    _check(*_moments(n, 1e-3), inject)
+
+
+@pytest.mark.parametrize("inject", [False, True])
+def test_every_code_through_the_queues(inject):
+    """Four iterations per workgroup whose codes are all left open, 512 to a
+    wavefront and iteration: the queues' rings of 1,024 entries wrap.  Every
+    preconditioner code is open at an eps below 1e-10; the injected uniforms
+    are 0 and every m a point of the grid, so that the momentum codes are too."""
+    n = (3 << 21) + 513
+    m, v = _moments(n, 1e-3)
+    u = None
+    if inject:
+        s_m = float(m.abs().max())
+        delta = np.log1p(s_m) / 32767.0
+        k = torch.randint(1, 32767, (n,), generator=torch.Generator().manual_seed(3))
+        grid = torch.expm1(k.double() * delta).float()
+        grid[0] = s_m
+        m = torch.copysign(grid, m)
+        u = (torch.zeros(n), torch.zeros(n))
+    print("case", n, inject, flush=True)
+    _check(m, v, inject, eps=1e-20, u=u)
 
 
 # S_m of about 0.05 (polynomials), 0.4 (atanh series), 40 (logarithm)
@@ -148,8 +185,18 @@ def test_moments_in_other_layouts():
                                          (0.1, 1e16, 1e-30)])
 @pytest.mark.parametrize("more", [0, 1, 2, 3])
 def test_every_code_decodes_exactly(s_m, s_v, eps, more):
-    print("case", s_m, s_v, eps, more, flush=True)
-    n = (1 << 16) + more
+    _check_decode((1 << 16) + more, s_m, s_v, eps)
+
+
+# a workgroup of export steps on above 2,097,152 elements
+@pytest.mark.parametrize("s_m,s_v,eps", [(1e-3, 1e-6, 1e-8), (0.5, 1e-2, 1e-8), (40.0, 100.0, 1e-8)])
+@pytest.mark.parametrize("n", [(1 << 21) + 3, (2 << 21) + 4097, 10500002])
+def test_codes_decode_exactly_over_several_iterations(n, s_m, s_v, eps):
+    _check_decode(n, s_m, s_v, eps)
+
+
+def _check_decode(n, s_m, s_v, eps):
+    print("case", n, s_m, s_v, eps, flush=True)
     codes = (torch.arange(n) & 0xFFFF).to(torch.int32).to(torch.int16)
     p = torch.nn.Parameter(torch.zeros(n, device=DEV))
     opt = LUMA([p], eps=eps)
