@@ -1,8 +1,10 @@
 """Tensors that start anywhere in memory (views of packed buckets or flat
 buffers, aligned to their elements only) step like aligned copies of them,
 bit for bit: the gradient, the parameter, the codes and injected uniforms,
-each at offsets of 0 to 7 elements, in every gradient type and on every
-route (small, one wavefront, workgroup, several chunks)."""
+each at offsets of 0 to 7 elements, in every gradient type: through the
+per-tensor op (one workgroup and several chunks), and through the optimizer
+the small tensors' route and the medium tensors' by workgroups (`split`) and
+by wavefronts."""
 
 import pytest
 import torch
@@ -58,16 +60,21 @@ def test_op_at_offsets(offsets, inject, dtype):
         assert _around(pb, p1, op) and _around(mb, m1, oq) and _around(wb, w1, oq + 1), n
 
 
+@pytest.mark.parametrize("split", [True, False])
 @pytest.mark.parametrize("dtype", TYPES)
-def test_optimizer_with_packed_gradients(dtype):
-    sizes = SIZES * 3 + [30001]
+def test_optimizer_with_packed_gradients(dtype, split):
+    """b's gradients, and every other parameter, lie off a 16-byte boundary."""
+    sizes = SIZES * 3 + [1537, 4609, 8191, 30001]
     gen = torch.Generator(device=DEV).manual_seed(5)
     a = [(torch.randn(n, device=DEV, generator=gen) * 0.02).requires_grad_(True) for n in sizes]
-    b = [p.detach().clone().requires_grad_(True) for p in a]
+    bufs = [_at(p.detach(), i % 4) for i, p in enumerate(a)]
+    b = [v.requires_grad_(True) for _, v in bufs]
     for p in a + b:
         p.grad_dtype = None
     oa, ob = LUMA(a, lr=1e-3), LUMA(b, lr=1e-3)
     ob._base_seed = oa._base_seed
+    for o in (oa, ob):
+        o._get_engine(a[0].device).split = split
     bucket = torch.zeros(sum(sizes) + 1, dtype=dtype, device=DEV)
     for q, g in zip(b, bucket[1:].split(sizes)):
         q.grad = g
@@ -77,6 +84,8 @@ def test_optimizer_with_packed_gradients(dtype):
             q.grad.copy_(p.grad)
         oa.step()
         ob.step()
+        assert oa._engine._wide == ob._engine._wide == split
+    assert all(_around(buf, v.detach(), i % 4) for i, (buf, v) in enumerate(bufs))
     sa, sb = oa.state_dict()["state"], ob.state_dict()["state"]
     for i, (p, q) in enumerate(zip(a, b)):
         assert torch.equal(p.detach(), q.detach()), i
