@@ -80,7 +80,8 @@ extern "C" {
 /*
  * Tensors above LUMA_SMALL_TENSOR and of at most this many elements are best
  * stepped one wavefront each (LumaStepArgs.medium_chunks): a whole
- * workgroup would leave most of its wavefronts idle on them.
+ * workgroup would leave most of its wavefronts idle on them.  (In a set that
+ * leaves the chip idle that costs nothing: LUMA_FLAG_SPLIT.)
  */
 #define LUMA_MEDIUM_TENSOR 8192
 

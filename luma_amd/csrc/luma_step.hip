@@ -3048,14 +3048,14 @@ int64_t luma_summary_words(int64_t numel, int32_t chunk_elems) {
 // four times faster and takes four times the slots.  Wavefronts -> wide, by
 // the tensors' elements (and workgroup records, split as below in either form):
 //                               257-512       1,025-2,048    4,097-8,192
-//   100                       26.2 -> 22.1   33.2 -> 22.7   66.8 -> 29.4
+//   100                       26.2 -> 22.4   33.2 -> 27.3   66.8 -> 29.4
 //   500                       22.9 -> 23.1   31.7 -> 28.2   77.3 -> 42.4
 //   700                       23.8 -> 25.7   33.7 -> 32.5   81.2 -> 52.6
 //   1,200                     30.7 -> 40.6   41.3 -> 48.3   95.1 -> 88.1
 //   2,000                     29.9 -> 51.3   44.8 -> 65.8  110.1 -> 126.7
 //   30, 100 records           31.1 -> 32.0   34.5 -> 31.7   73.2 -> 33.8
-//   100, 100 records          31.2 -> 35.6   35.2 -> 34.7   75.1 -> 42.1
-//   300, 300 records          51.2 -> 57.5   53.5 -> 58.5   91.6 -> 62.6
+//   100, 100 records          31.2 -> 34.4   35.2 -> 34.7   75.1 -> 42.1
+//   300, 300 records          51.2 -> 57.5   53.5 -> 58.5   95.6 -> 62.6
 //   300, 800 records          96.7 -> 97.3   97.2 -> 100.2 134.2 -> 105.1
 //   1,000, 800 records        99.2 -> 101.4 104.8 -> 107.6 154.0 -> 136.4
 // So the tensors may be as many as their length pays for: alone (with small
@@ -3066,16 +3066,16 @@ int64_t luma_summary_words(int64_t numel, int32_t chunk_elems) {
 // the workgroups are one round: parts of 8,192 elements while there are at
 // most 816, of 4,096 at most 768, of 2,048 at most 384 (with more, pass 1 and
 // finalize lose what pass 2 gains).  By the part's length, 16,384 / 8,192 /
-// 4,096 / 2,048 elements:
-//   50 records                  40.0  31.0  26.4  26.3
-//   100 records                 44.2  34.0  31.1  30.3
-//   200 records                 45.5  41.8  40.0
-//   340 records                 59.4  52.3  56.7
-//   400 records                 60.3  59.9
-//   500 records                 62.7  66.9
+// 4,096 / 2,048 elements (and six short tensors in wavefronts):
+//   20 records                  40.5  32.2  25.8  23.6
+//   50 records                  42.2  33.2  26.7  25.7
+//   100 records                 41.8  34.3  30.9  35.3
+//   200 records                 44.1  41.2  42.1
+//   300 records                 56.3  50.7  54.1
+//   400 records                 58.3  59.3
 // Medium tensors' wavefronts come after the parts; where they are long, only
 // parts that leave them CUs of their own (256) are worth it: 100 records and
-// 100 tensors of 1,025-2,048 elements 42.0, 34.0, 36.8, 43.2.
+// 100 tensors of 1,025-2,048 elements 43.2, 35.2, 39.7, 46.0.
 // A wide medium tensor fills one part or a few of its record's; workgroups go
 // to the eight XCDs in turn, so the others lie idle: its tensors' first parts
 // have the 256 >> split CUs of every second, fourth or eighth XCD's turn.

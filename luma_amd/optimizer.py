@@ -359,7 +359,8 @@ class _Engine:
         Tensors of at most SMALL_TENSOR elements are stepped a wavefront per
         chunk by the exact kernels, and those above it and of at most
         MEDIUM_TENSOR elements (and one chunk) one wavefront each by the fast
-        kernels, four to a workgroup; each run is ordered largest first, so the four
+        kernels, four to a workgroup (or, in a small set, a workgroup each:
+        _split_plan); each run is ordered largest first, so the four
         wavefronts of a small-tensor workgroup step tensors of about one size
         and every launch ends on its shortest work.  The others keep their
         order, unless there are STEP_TARGET_CHUNKS of them or more (chunk_for
@@ -954,8 +955,10 @@ class LUMA(Optimizer):
         # code summaries: SUMMARY_WORDS words per chunk at this step's chunk length
         chunk = engine.summary_chunk(np.fromiter((w[2].numel() for w in work), dtype=np.int64,
                                                  count=len(work)))
-        # (a tensor below one whole 2048-element iteration, or stepped by a
-        # single wavefront, never reads a summary: it gets none)
+        # (a tensor below one whole 2048-element iteration never reads a summary,
+        # nor does one that a single wavefront steps: it gets none.  Where a
+        # small set gives such tensors a workgroup each they go without too:
+        # their codes are few, and the next step's set may be a larger one)
         least = max(_SUMMARY_MIN, engine._wave_limit() + 1)
         no_summ = [(self.state[w[1]], w[2]) for w in work
                    if w[2].numel() >= least and (
